@@ -158,6 +158,21 @@ def test_decode_few_long_sequences(lens):
             assert int(out[i].abs().sum()) == 0
 
 
+@pytest.mark.parametrize("lens", [[1], [63], [64], [65], [81, 0, 16], [33] * 3 + [2049], [7] * 63 + [6000],
+                                  [7] * 64 + [6000], [0] * 60 + [300] * 4, [0] * 61 + [300] * 4],
+                         ids=["1", "63", "64", "65", "81+0+16", "3x33+2049", "64 seqs", "65 seqs", "64 with empty rows",
+                              "65 with empty rows"])
+def test_decode_merge_forms(lens):
+    """The merge with four workgroups per sequence (up to 64 sequences) and with one (beyond), over one partial, as many
+    as a wave takes in a batch and more (6000 tokens in up to 62 ranges), and ranges of four 16-token steps and fewer."""
+    gen = torch.Generator().manual_seed(90 + len(lens) + lens[0])
+    kc, vc, tables = paged_pool(gen, [max(n, 1) for n in lens], sum(-(-max(n, 1) // BLOCK) for n in lens) + 2)
+    (_, _), out = _check(randn(gen, len(lens), H, D), kc, vc, lens, tables, f"{len(lens)} sequences")
+    for i, n in enumerate(lens):
+        if n == 0:
+            assert int(out[i].abs().sum()) == 0
+
+
 def test_decode_repeated_calls_of_changing_batch():
     """Back-to-back calls that reuse the workspace with different batch sizes and split counts."""
     gen = torch.Generator().manual_seed(36)

@@ -73,12 +73,14 @@ __device__ __forceinline__ void copy_new_rows(const DecodeArgs& p, int wid) {
 // workgroups touching b, g_first..g_last in merge_row, each left a partial at slot b + g. Online rescale over the
 // partials (fp32), the loads of kMergeBatch partials in flight together. Runs after decode_kernel on the same stream,
 // which makes the partials visible. In varlen store mode workgroups past the sequences copy the step's new rows into
-// the caches (copy_new_rows).
+// the caches (copy_new_rows). PG workgroups per sequence, 16 / PG heads each (merge_row).
+template <int PG>
 __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs p) {
-  const int b = blockIdx.x;
+  __shared__ __attribute__((aligned(16))) float comb[PG > 1 ? PG - 1 : 1][kWave][12];
+  const int b = blockIdx.x / PG, part = blockIdx.x % PG;
   const int tid = threadIdx.x;
   if (b >= p.batch) {  // (workgroup-uniform) a copy workgroup of the varlen store mode
-    copy_new_rows(p, b - p.batch);
+    copy_new_rows(p, (int)blockIdx.x - PG * p.batch);
     return;
   }
   int s_tot = p.steps[p.batch], s_b = p.steps[b], s_e = p.steps[b + 1], s_g = p.steps[p.batch + 1];
@@ -87,7 +89,8 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs p) {
     c0 = p.cu_q[b];
     c1 = p.cu_q[b + 1];
   }
-  const bool own_row = p.slot_mapping && !p.cu_q;  // store mode: this sequence's row (varlen: the copy workgroups)
+  // store mode: this sequence's row (varlen: the copy workgroups)
+  const bool own_row = p.slot_mapping && !p.cu_q && part == 0;
   if (own_row) slot32 = p.slot_mapping[b];
   // every value in registers here: the loads go out together, one round trip (left to itself the compiler sinks
   // each load to its first use, behind the branches, one round trip apiece)
@@ -108,15 +111,18 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeArgs p) {
       kv_chunk = ld_g16(src + chunk * 8);
     }
   }
-  merge_row(p, b, tid, s_tot, s_b, s_e, s_g, c0, c1);
+  merge_row<PG>(p, b, part, tid, s_tot, s_b, s_e, s_g, c0, c1, comb);
   if (kv_dst) __builtin_nontemporal_store(kv_chunk, reinterpret_cast<u32x4*>(kv_dst));
 }
 
 }  // namespace
 
 hipError_t launch_decode_merge(const DecodeArgs& a, hipStream_t stream) {
-  const int64_t wgs = (int64_t)a.batch + (a.slot_mapping && a.cu_q && a.copy_rows > 0 ? a.copy_wgs : 0);
-  decode_merge_kernel<<<dim3((unsigned)wgs), dim3(256), 0, stream>>>(a);
+  const int64_t copies = a.slot_mapping && a.cu_q && a.copy_rows > 0 ? a.copy_wgs : 0;
+  if (a.batch <= kMergeSplitBatch)
+    decode_merge_kernel<4><<<dim3((unsigned)(4 * a.batch + copies)), dim3(256), 0, stream>>>(a);
+  else
+    decode_merge_kernel<1><<<dim3((unsigned)(a.batch + copies)), dim3(256), 0, stream>>>(a);
   return hipGetLastError();
 }
 

@@ -55,16 +55,21 @@ constexpr int kThreads = kWaves * kWave;
 // The work is balanced in units of one wave tile: with 64-token units a config-4 launch (2700 units over 256
 // workgroups) gave some workgroups 11 units and others 10, and the 11-unit ones (10 % more bytes) ended the launch.
 constexpr int kMaxHeads = 16;
-#ifndef VOX_MAX_PIECES
-#define VOX_MAX_PIECES 32
-#endif
 #ifndef VOX_MERGE_BATCH
 #define VOX_MERGE_BATCH 8
 #endif
 // Most partials one sequence is cut into. A sequence of n steps meets at most about n G / S + 2 of G equal ranges of
-// S steps, so a launch uses G' = min(grid, (kMaxPieces - 2) S / n_max) workgroups (the others leave after the layout
+// S steps, so a launch uses G' = min(grid, S / 4, (kMaxPieces - 2) S / n_max) workgroups (the others leave after the layout
 // scan): a long sequence among few is not cut into one-step pieces, each a partial for the merge kernel to load.
-constexpr int kMaxPieces = VOX_MAX_PIECES;
+// Batches whose merge has four workgroups per sequence take twice the pieces (one stream of 4000 tokens: 13.7 us a layer
+// with 32, 12.9 with 64).
+constexpr int kMaxPieces = 32;
+constexpr int kMaxPiecesSplit = 64;
+// Batches of up to this many sequences merge with four workgroups per sequence (merge_row<4>), a quarter of the partials
+// per wave; beyond, the sequences' own workgroups fill the CUs. A layer of a step, one workgroup against four: 1 stream
+// of 420 tokens 12.0 -> 10.0 us, 13 of 2500-4096 19.9 -> 16.9, 40 of 200-1500 17.2 -> 16.1; 80 of 100-1024 18.0 -> 18.4,
+// 150 of 256-2048 37.6 -> 38.4, 256 of 50-1024 33.8 -> 35.3.
+constexpr int kMergeSplitBatch = 64;
 constexpr int kMergeBatch = VOX_MERGE_BATCH;  // partials whose loads the merge kernel keeps in flight together
 constexpr int kMOff = kMaxHeads * kD;          // inside a partial: O [16 heads][128], then m[16], l[16] (log2 domain)
 constexpr int kLOff = kMOff + kMaxHeads;
@@ -143,10 +148,13 @@ __device__ __forceinline__ int64_t muldiv(int64_t a, int64_t b, int64_t c, int64
   return (int64_t)(num / (uint64_t)d);
 }
 
-// G' of a launch over `steps` steps whose longest sequence has `max_seq_steps`; at most `steps`, so no range is empty
-__device__ __forceinline__ int active_workgroups(int grid, int64_t steps, int max_seq_steps) {
+// G' of a launch over `steps` steps whose longest sequence has `max_seq_steps`: at most one workgroup per kWaves steps (a
+// range of fewer leaves waves idle, takes as long, and adds a partial to merge: one stream of 420 tokens, 27 ranges of a
+// step each take 12.0 us a layer with their merge, 7 of four 10.0), so no range is empty
+__device__ __forceinline__ int active_workgroups(int grid, int64_t steps, int max_seq_steps, int batch) {
   if (max_seq_steps <= 0) return 1;
-  const int64_t cap = min(steps, muldiv(kMaxPieces - 2, steps, 0, max_seq_steps));
+  const int pieces = batch <= kMergeSplitBatch ? kMaxPiecesSplit : kMaxPieces;
+  const int64_t cap = min((steps + kWaves - 1) / kWaves, muldiv(pieces - 2, steps, 0, max_seq_steps));
   return (int)max((int64_t)1, min((int64_t)grid, cap));
 }
 
@@ -446,7 +454,7 @@ __device__ __forceinline__ void decode_split(const DecodeArgs& p, const int g, c
     if (tid == 0) L.start[p.batch] = run;
     __syncthreads();
     S = uniform(run);
-    G = active_workgroups(grid, S, uniform(nmax));
+    G = active_workgroups(grid, S, uniform(nmax), p.batch);
     if (g == 0) {  // the layout decode_merge_kernel reads, then the active workgroup count (a record keeps it)
       for (int i = tid; i <= p.batch; i += kThreads) p.steps[i] = L.start[i];
       if (tid == 0) p.steps[p.batch + 1] = G;
@@ -728,20 +736,25 @@ __device__ __forceinline__ void decode_split(const DecodeArgs& p, const int g, c
   }
 }
 
-// The merge of sequence b's split-KV partials into its output row (decode_merge_kernel).
+// The merge of sequence b's split-KV partials into its output row (decode_merge_kernel), heads [16 / PG part,
+// 16 / PG (part + 1)) of it by one workgroup of 256 threads. PG = 1: thread (head, 8 dims) takes every partial in turn.
+// PG = 4: wave w takes partials w, w + 4, ... of 4 heads and the waves combine theirs in `comb` (LDS): a quarter of the
+// serial loads, and the row's partials read by four CUs instead of one.
 // steps: the layout's total S, sequence b's first and end steps sb, eb, and the active workgroups G (with S >= 1, none
 // has an empty range); [c0, c1): b's query rows (b's row alone outside varlen mode).
-__device__ __forceinline__ void merge_row(const DecodeArgs& p, int b, int tid, int64_t S, int64_t sb, int64_t eb,
-                                          int64_t G, int c0, int c1) {
-  const int hh = tid >> 4;
+template <int PG>
+__device__ __forceinline__ void merge_row(const DecodeArgs& p, int b, int part, int tid, int64_t S, int64_t sb,
+                                          int64_t eb, int64_t G, int c0, int c1, float (*comb)[kWave][12]) {
+  const int pg = PG == 1 ? 0 : tid >> 6;  // wave-uniform
+  const int hh = PG == 1 ? tid >> 4 : part * (kMaxHeads / PG) + ((tid & 63) >> 4);
   const int d0 = (tid & 15) * 8;
   const int H = p.num_heads;
   const int64_t row = c0;
   if (c1 - c0 != 1) return;  // varlen mode: not a one-query row, the prefill kernel writes it
   uint16_t* ob = p.out + row * p.out_row_stride + (int64_t)hh * kD + d0;
-  if (hh >= H) return;
+  const bool writes = hh < H && pg == 0;
   if (eb == sb) {  // empty (padded) row: defined zeros
-    *reinterpret_cast<u32x4*>(ob) = zero4();
+    if (writes) *reinterpret_cast<u32x4*>(ob) = zero4();
     return;
   }
   const int g_first = (int)muldiv(sb + 1, G, S - 1, S) - 1;
@@ -752,7 +765,20 @@ __device__ __forceinline__ void merge_row(const DecodeArgs& p, int b, int tid, i
   float o2[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) o2[i] = 0.f;
-  for (int g0 = g_first; g0 <= g_last; g0 += kMergeBatch) {
+  auto fold = [&](float mc, float lc, const f32x4& oa, const f32x4& ob4) {
+    const float mn = fmaxf(M2, mc);
+    const float mu = mn == -INFINITY ? 0.f : mn;
+    const float a = fast_exp2(M2 - mu);
+    const float e = fast_exp2(mc - mu);
+    L2 = L2 * a + e * lc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o2[i] = o2[i] * a + e * oa[i];
+      o2[i + 4] = o2[i + 4] * a + e * ob4[i];
+    }
+    M2 = mn;
+  };
+  for (int g0 = g_first + pg; g0 <= g_last; g0 += PG * kMergeBatch) {
     float mc[kMergeBatch], lc[kMergeBatch];
     f32x4 oa[kMergeBatch], obv[kMergeBatch];
 #pragma unroll
@@ -760,9 +786,8 @@ __device__ __forceinline__ void merge_row(const DecodeArgs& p, int b, int tid, i
       mc[u] = -INFINITY;
       lc[u] = 0.f;
       oa[u] = obv[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      // loads only up to the sequence's last range: the condition is workgroup-uniform, so the slots past it
-      // cost no traffic
-      const int64_t gg = g0 + u;
+      // loads only up to the sequence's last range: the condition is wave-uniform, so the slots past it cost no traffic
+      const int64_t gg = g0 + PG * u;
       if (gg <= g_last) {
         const float* pc = p.partials + (b + gg) * kPartialFloats;
         mc[u] = pc[kMOff + hh];
@@ -772,20 +797,24 @@ __device__ __forceinline__ void merge_row(const DecodeArgs& p, int b, int tid, i
       }
     }
 #pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
-      const float mn = fmaxf(M2, mc[u]);
-      const float mu = mn == -INFINITY ? 0.f : mn;
-      const float a = fast_exp2(M2 - mu);
-      const float e = fast_exp2(mc[u] - mu);
-      L2 = L2 * a + e * lc[u];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        o2[i] = o2[i] * a + e * oa[u][i];
-        o2[i + 4] = o2[i + 4] * a + e * obv[u][i];
-      }
-      M2 = mn;
-    }
+    for (int u = 0; u < kMergeBatch; ++u) fold(mc[u], lc[u], oa[u], obv[u]);
   }
+  if constexpr (PG > 1) {
+    const int lane = tid & 63;
+    if (pg > 0) {
+      *reinterpret_cast<f32x4*>(&comb[pg - 1][lane][0]) = f32x4{o2[0], o2[1], o2[2], o2[3]};
+      *reinterpret_cast<f32x4*>(&comb[pg - 1][lane][4]) = f32x4{o2[4], o2[5], o2[6], o2[7]};
+      comb[pg - 1][lane][8] = M2;
+      comb[pg - 1][lane][9] = L2;
+    }
+    __syncthreads();
+    if (pg > 0) return;
+#pragma unroll
+    for (int u = 0; u < PG - 1; ++u)
+      fold(comb[u][lane][8], comb[u][lane][9], *reinterpret_cast<const f32x4*>(&comb[u][lane][0]),
+           *reinterpret_cast<const f32x4*>(&comb[u][lane][4]));
+  }
+  if (!writes) return;
   const float inv = L2 > 0.f ? 1.f / L2 : 0.f;
   *reinterpret_cast<u32x4*>(ob) =
       u32x4{pack_bf16x2(o2[0] * inv, o2[1] * inv), pack_bf16x2(o2[2] * inv, o2[3] * inv),

@@ -335,3 +335,23 @@ def test_prefill_store_paged_rejects_bad_arguments_before_launching():
     empty = list(args)
     empty[17], empty[7] = 0, 0  # no sequences, no rows
     assert lib.vox_prefill_attn_store_paged(*empty) == _lib.VOX_OK
+
+
+def test_calls_module_takes_what_ctypes_takes():
+    """The CPython entries of the hot calls (csrc/host_calls.cpp) against the ctypes functions of a second handle on the
+    library: pointers as addresses, None or ctypes objects, integers reduced to the C type, any argument the library
+    rejects, a wrong number of arguments."""
+    lib, plain = _lib.load(), ctypes.CDLL(_lib.LIB_PATH)
+    fn = plain.vox_store_kvcache
+    fn.restype, fn.argtypes = _lib._SIGNATURES["vox_store_kvcache"]
+    for p in (None, 16, 8, ctypes.c_void_p(16), ctypes.c_void_p(None)):
+        for args in ((p, 16, 256, 256, 16, 16, 10, 16, 0, 2, 128, None), (16, p, 100, 256, 16, 16, 10, 16, 4, 2, 128, 0),
+                     (16, 16, 256, 256, p, 16, 0, 16, 4, 2, 128, None), (16, 16, 256, 256, 16, p, 10, 16, -1, 2, 128, None),
+                     (p, 16, 256, 256, 16, 16, 0, 16, 2 ** 64, (1 << 32) + 2, 128, None)):
+            assert lib.vox_store_kvcache(*args) == fn(*args), args
+    size = plain.vox_prefill_int8_workspace_bytes
+    size.restype, size.argtypes = _lib._SIGNATURES["vox_prefill_int8_workspace_bytes"]
+    for args in ((4096, 16, 256, 16, 2, 128, 1), (7, 1, 7, 16, 2, 128, 1), (2304, 8, 512, 16, 2, 128, True)):
+        assert lib.vox_prefill_int8_workspace_bytes(*args) == size(*args)
+    with pytest.raises(TypeError):
+        lib.vox_store_kvcache(None)

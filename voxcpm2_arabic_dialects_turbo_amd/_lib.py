@@ -111,6 +111,16 @@ def load() -> ctypes.CDLL:
                 fn.argtypes = args
             if lib.vox_abi_version() != ABI_VERSION:
                 raise VoxAttnError(f"libvoxattn ABI {lib.vox_abi_version()} != {ABI_VERSION}: rebuild the library")
+            # the entry points called on every layer, through the CPython module: the same functions, without ctypes'
+            # argument conversion
+            try:
+                from . import _calls
+            except ImportError as e:
+                raise VoxAttnError(f"_calls.so ({e}): run `python -m voxcpm2_arabic_dialects_turbo_amd.build`") from e
+            fast = [n for n in EXPORTS if hasattr(_calls, n)]
+            _calls.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in fast})
+            for n in fast:
+                setattr(lib, n, getattr(_calls, n))
             _lib = lib
     return _lib
 
@@ -126,7 +136,17 @@ def check(status: int, what: str) -> None:
 
 def stream_handle(device: torch.device) -> int:
     """The hipStream_t of torch's current stream on ``device`` (0 = null stream)."""
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
+
+
+def _raw_stream(index: int) -> int:
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# torch's current stream as a handle, without a Stream object around it (0.1 us against 3), where this torch has it
+if hasattr(torch._C, "_cuda_getCurrentRawStream"):
+    _raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 _capture_info = None

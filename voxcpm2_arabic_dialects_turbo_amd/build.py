@@ -1,7 +1,8 @@
 """Builds libvoxattn.so in-tree with hipcc for gfx950 (run as ``python -m voxcpm2_arabic_dialects_turbo_amd.build``).
 
 The attention library is one shared library, C ABI only (include/vox_attn.h): no torch headers, no pybind. The
-sources compile in parallel and link into ``voxcpm2_arabic_dialects_turbo_amd/libvoxattn.so``. Beside it,
+sources compile in parallel and link into ``voxcpm2_arabic_dialects_turbo_amd/libvoxattn.so``. Beside it, ``_calls.so`` is
+the CPython module through which the operators call it (csrc/host_calls.cpp, host code only), and
 ``libvoxprobe.so`` (include/vox_probe.h) holds the memory-rate probes bench.py runs; the attention path never loads
 it. Packed FP32 VALU instructions are disabled for
 device code (``-packed-fp32-ops``); hipcc's host pass warns that it does not know that feature, which is harmless.
@@ -13,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -24,6 +26,9 @@ LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 SOURCES = ["store_kvcache.hip", "decode_attn.hip", "prefill_attn.hip", "quantize_rows.hip", "kv_copy.hip", "capi.hip"]
 PROBE_PATH = os.path.join(PKG_DIR, "libvoxprobe.so")
 PROBE_SOURCES = ["bench_probe.hip"]
+# the CPython entry to the C ABI (host code only)
+CALLS_PATH = os.path.join(PKG_DIR, "_calls.so")
+CALLS_SOURCE = "host_calls.cpp"
 ARCH = "gfx950"
 
 
@@ -77,6 +82,10 @@ def build(verbose: bool = False) -> str:
         tmp = path + ".tmp"
         _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])
         os.replace(tmp, path)
+    cxx = os.environ.get("CXX") or shutil.which("g++") or cc
+    _run([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
+          f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, CALLS_SOURCE), "-o", CALLS_PATH + ".tmp"])
+    os.replace(CALLS_PATH + ".tmp", CALLS_PATH)
     return LIB_PATH
 
 

@@ -28,11 +28,24 @@ def _require(cond: bool, msg: str) -> None:
 
 
 def _check_cuda(*tensors: torch.Tensor) -> torch.device:
-    dev = tensors[0].device
+    index = tensors[0].get_device()  # -1: not on a GPU
     for t in tensors:
-        if t is not None and (t.device.type != "cuda" or t.device != dev):
-            raise ValueError(f"all tensors must be on the same GPU, got {t.device} and {dev}")
-    return dev
+        if t is not None and (t.get_device() != index or index < 0):
+            raise ValueError(f"all tensors must be on the same GPU, got {t.device} and {tensors[0].device}")
+    return tensors[0].device
+
+
+def _flat(t: torch.Tensor) -> torch.Tensor:
+    return t if t.dim() == 1 else t.reshape(-1)
+
+
+def _smooth(inv_smooth: torch.Tensor, n: int) -> torch.Tensor:
+    """inv_smooth as n contiguous fp32 values."""
+    if inv_smooth.numel() != n:
+        raise ValueError(f"inv_smooth must hold H * head_dim = {n} values")
+    if inv_smooth.dtype == torch.float32 and inv_smooth.dim() == 1 and inv_smooth.is_contiguous():
+        return inv_smooth
+    return inv_smooth.reshape(-1).to(torch.float32).contiguous()
 
 
 def _as_i32(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -67,7 +80,7 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
         raise ValueError("store_kvcache: caches must be contiguous [num_blocks, block_size, HK, head_dim]")
     if k_cache.shape != v_cache.shape:
         raise ValueError(f"store_kvcache: k_cache {tuple(k_cache.shape)} and v_cache {tuple(v_cache.shape)} differ")
-    slots = _as_i32(slot_mapping.reshape(-1), "slot_mapping")
+    slots = _as_i32(_flat(slot_mapping), "slot_mapping")
     lib = _lib.load()
     _lib.check(lib.vox_store_kvcache(key.data_ptr(), value.data_ptr(), key.stride(0), value.stride(0),
                                      k_cache.data_ptr(), v_cache.data_ptr(), k_cache.numel() // D, slots.data_ptr(),
@@ -195,7 +208,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         q = q.contiguous()
     bt = block_tables if (block_tables.dtype == torch.int32 and block_tables.stride(1) == 1) else \
         _as_i32(block_tables, "block_tables")
-    lens = _as_i32(context_lens.reshape(-1), "context_lens")
+    lens = _as_i32(_flat(context_lens), "context_lens")
     max_blocks = bt.shape[1]
     lib = _lib.load()
     ws = decode_workspace(dev)
@@ -216,7 +229,7 @@ def decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
         raise ValueError("decode store: key/value heads must be contiguous")
     if slot_mapping.numel() != B:
         raise ValueError("decode store: slot_mapping must hold one slot per sequence")
-    slots = _as_i32(slot_mapping.reshape(-1), "slot_mapping")
+    slots = _as_i32(_flat(slot_mapping), "slot_mapping")
     _lib.check(lib.vox_decode_attn_store(q.data_ptr(), q.stride(0), key.data_ptr(), value.data_ptr(), key.stride(0),
                                          value.stride(0), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                                          num_blocks, block_size, bt.data_ptr(), bt.stride(0), max_blocks,
@@ -255,9 +268,7 @@ def varlen_attention(q: torch.Tensor, k: torch.Tensor | None, v: torch.Tensor | 
         out_scale = torch.empty(T, dtype=torch.float32, device=dev)
         if inv_smooth is not None:
             _check_cuda(q, inv_smooth)
-            if inv_smooth.numel() != H * D:
-                raise ValueError(f"inv_smooth must hold H * head_dim = {H * D} values")
-            inv_smooth = inv_smooth.reshape(-1).to(torch.float32).contiguous()
+            inv_smooth = _smooth(inv_smooth, H * D)
         out = (out_q, out_scale)
     elif out is None:
         out = torch.empty(T, H, D, dtype=q.dtype, device=dev)
@@ -358,16 +369,17 @@ def prefill_attention_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k
     Reference: the prefill branch of nanovllm_voxcpm/model/layers.py:326-348."""
     T, H, D = q.shape
     N, HK, Dk = k.shape
-    _require(k.stride(-1) == 1 and v.stride(-1) == 1, "key/value: last dim must be contiguous")
-    _require(k.stride(1) == Dk and v.stride(1) == Dk, "key/value: heads must be head_dim apart")
+    qs, ks, vs = q.stride(), k.stride(), v.stride()
+    _require(ks[-1] == 1 and vs[-1] == 1, "key/value: last dim must be contiguous")
+    _require(ks[1] == Dk and vs[1] == Dk, "key/value: heads must be head_dim apart")
     _require(k_cache.stride(1) == HK * Dk and v_cache.stride(1) == HK * Dk,
              "caches: slot rows must be num_kv_heads*head_dim apart")
     _require(slot_mapping.numel() == N, "slot_mapping must hold one slot per token")
     dev = _check_cuda(q, k, v, k_cache, v_cache, slot_mapping, cu_seqlens_q, cu_seqlens_k)
-    if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16 \
-            or k_cache.dtype != torch.bfloat16 or v_cache.dtype != torch.bfloat16:
+    bf16 = torch.bfloat16
+    if q.dtype != bf16 or k.dtype != bf16 or v.dtype != bf16 or k_cache.dtype != bf16 or v_cache.dtype != bf16:
         raise TypeError("prefill_attention_store takes bf16 q, k, v and caches")
-    if D != HEAD_DIM or Dk != HEAD_DIM or q.stride(2) != 1 or q.stride(1) != D or v.shape != k.shape:
+    if D != HEAD_DIM or Dk != HEAD_DIM or qs[2] != 1 or qs[1] != D or v.shape != k.shape:
         raise ValueError(f"q / k / v must be [T, H, {HEAD_DIM}] / [N, HK, {HEAD_DIM}] with contiguous heads")
     if not (k_cache.is_contiguous() and v_cache.is_contiguous()) or k_cache.shape != v_cache.shape:
         raise ValueError("caches must be contiguous [num_blocks, block_size, HK, head_dim] of one shape")
@@ -378,7 +390,7 @@ def prefill_attention_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k
         raise ValueError("cu_seqlens_k must have as many entries as cu_seqlens_q")
     cu_q = _as_i32(cu_seqlens_q, "cu_seqlens_q")
     cu_k = _as_i32(cu_seqlens_k, "cu_seqlens_k")
-    slots = _as_i32(slot_mapping.reshape(-1), "slot_mapping")
+    slots = _as_i32(_flat(slot_mapping), "slot_mapping")
     lib = _lib.load()
     bt = None
     if block_table is not None:
@@ -397,13 +409,11 @@ def prefill_attention_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k
         out_scale = torch.empty(T, dtype=torch.float32, device=dev)
         if inv_smooth is not None:
             _check_cuda(q, inv_smooth)
-            if inv_smooth.numel() != H * D:
-                raise ValueError(f"inv_smooth must hold H * head_dim = {H * D} values")
-            inv_smooth = inv_smooth.reshape(-1).to(torch.float32).contiguous()
+            inv_smooth = _smooth(inv_smooth, H * D)
         ws_bytes = lib.vox_prefill_int8_workspace_bytes(T, max(B, 0), int(max_seqlen_q), H, HK, D, 1 if causal else 0)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
         _lib.check(lib.vox_prefill_attn_int8_store(
-            q.data_ptr(), q.stride(0), k.data_ptr(), v.data_ptr(), k.stride(0), v.stride(0), slots.data_ptr(), N,
+            q.data_ptr(), qs[0], k.data_ptr(), v.data_ptr(), ks[0], vs[0], slots.data_ptr(), N,
             k_cache.data_ptr(), v_cache.data_ptr(), num_blocks, block_size, None if bt is None else bt.data_ptr(),
             0 if bt is None else bt.stride(0), 0 if bt is None else bt.shape[1], cu_q.data_ptr(), cu_k.data_ptr(),
             max(B, 0), int(max_seqlen_q) if T else 0, H, HK, D, float(softmax_scale), 1 if causal else 0,
@@ -423,14 +433,14 @@ def prefill_attention_store(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k
                 plan = getattr(_SCOPE, "key", None)
             mode = _plan_mode(dev, plan, "varlen-store", B, int(bt.shape[1]), H, HK, int(block_size))
         _lib.check(lib.vox_prefill_attn_store_paged(
-            q.data_ptr(), q.stride(0), k.data_ptr(), v.data_ptr(), k.stride(0), v.stride(0), slots.data_ptr(), N,
+            q.data_ptr(), qs[0], k.data_ptr(), v.data_ptr(), ks[0], vs[0], slots.data_ptr(), N,
             k_cache.data_ptr(), v_cache.data_ptr(), num_blocks, block_size, bt.data_ptr(), bt.stride(0), bt.shape[1],
             cu_q.data_ptr(), cu_k.data_ptr(), max(B, 0), int(max_seqlen_q) if T else 0, H, HK, D, float(softmax_scale),
             1 if causal else 0, out.data_ptr(), out.stride(0), mode, None if ws is None else ws.data_ptr(),
             0 if ws is None else ws.numel(), _lib.stream_handle(dev)), "prefill_attn_store_paged")
         return out
-    _lib.check(lib.vox_prefill_attn_store(q.data_ptr(), q.stride(0), k.data_ptr(), v.data_ptr(), k.stride(0),
-                                          v.stride(0), slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+    _lib.check(lib.vox_prefill_attn_store(q.data_ptr(), qs[0], k.data_ptr(), v.data_ptr(), ks[0],
+                                          vs[0], slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                                           k_cache.numel() // (HK * Dk), N, cu_q.data_ptr(), cu_k.data_ptr(), max(B, 0),
                                           int(max_seqlen_q) if T else 0, H, HK, D, float(softmax_scale),
                                           1 if causal else 0, out.data_ptr(), out.stride(0), _lib.stream_handle(dev)),

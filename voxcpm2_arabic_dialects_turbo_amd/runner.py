@@ -27,6 +27,7 @@ they touch. The arrays are written straight into a page-locked staging buffer la
 from __future__ import annotations
 
 import math
+from itertools import chain
 from dataclasses import dataclass, field
 from typing import Iterable, Sequence
 
@@ -61,7 +62,9 @@ _ALIGN = 256  # every array starts at a multiple of 256 bytes, as separate devic
 @dataclass
 class _Slot:
     host: torch.Tensor | None = None   # page-locked uint8 buffer
+    raw: np.ndarray | None = None      # ... as numpy
     done: object = None                # CUDA event recorded after the copy out of ``host``
+    pending: bool = False              # the event has been recorded and not yet waited for
 
 
 @dataclass
@@ -80,40 +83,35 @@ class StepStaging:
     _turn: int = 0
     _host: torch.Tensor | None = None
     _slot: _Slot | None = None
-    _parts: list[tuple[int, np.dtype, tuple]] = field(default_factory=list)
+    _parts: list[tuple[int, np.dtype, tuple, int]] = field(default_factory=list)
     _used: int = 0
 
     def layout(self, specs: Sequence[tuple[np.dtype, tuple]]) -> list[np.ndarray]:
         """Reserves one array per (dtype, shape) and returns writable numpy views of them (contents undefined)."""
         dev = torch.device(self.device)
-        offsets, end = [], 0
+        parts, end = [], 0
         for dtype, shape in specs:
             dtype = np.dtype(dtype)
-            offsets.append(end)
-            end += -(-(dtype.itemsize * math.prod(shape)) // _ALIGN) * _ALIGN
+            n = math.prod(shape)
+            parts.append((end, dtype, shape, n))
+            end += -(-(dtype.itemsize * n) // _ALIGN) * _ALIGN
         need = max(end, _ALIGN)
         persistent = dev.type == "cuda" and not torch.cuda.is_current_stream_capturing()
         if persistent:
             slot = self._slots[self._turn]
             self._turn ^= 1
-            if slot.done is not None:
+            if slot.done is not None and slot.pending:
                 slot.done.synchronize()
-                slot.done = None
+                slot.pending = False
             if slot.host is None or slot.host.numel() < need:
                 slot.host = torch.empty(2 * need, dtype=torch.uint8, pin_memory=True)
-            self._host, self._slot = slot.host, slot
+                slot.raw = slot.host.numpy()
+            self._host, self._slot, raw = slot.host, slot, slot.raw
         else:
             self._host = torch.empty(need, dtype=torch.uint8, pin_memory=dev.type == "cuda")
-            self._slot = None
-        raw = self._host.numpy()
-        self._parts, self._used = [], need
-        views = []
-        for off, (dtype, shape) in zip(offsets, specs):
-            dtype = np.dtype(dtype)
-            n = math.prod(shape)
-            views.append(raw[off:off + n * dtype.itemsize].view(dtype).reshape(shape))
-            self._parts.append((off, dtype, tuple(shape)))
-        return views
+            self._slot, raw = None, self._host.numpy()
+        self._parts, self._used = parts, need
+        return [np.ndarray(shape, dtype, raw, off) for off, dtype, shape, _ in parts]
 
     def upload(self) -> list[torch.Tensor]:
         """One copy of the laid-out bytes to the device (non-blocking from page-locked memory); the views."""
@@ -122,16 +120,21 @@ class StepStaging:
         if dev.type == "cuda":
             dst = src.to(dev, non_blocking=True)
             if self._slot is not None:
-                ev = torch.cuda.Event()
-                ev.record()
-                self._slot.done = ev
+                if self._slot.done is None:
+                    self._slot.done = torch.cuda.Event()
+                self._slot.done.record()
+                self._slot.pending = True
         else:
             dst = src.clone()
+        typed = {}  # the device copy as one tensor per element type; the arrays are slices of them
         out = []
-        for off, dtype, shape in self._parts:
-            n = math.prod(shape)
-            t = dst[off:off + n * dtype.itemsize].view(_TORCH_DTYPE[dtype])
-            out.append(t.view(shape))
+        for off, dtype, shape, n in self._parts:
+            t = typed.get(dtype)
+            if t is None:
+                t = typed[dtype] = dst.view(_TORCH_DTYPE[dtype])
+            at = off // dtype.itemsize
+            t = t[at:at + n]
+            out.append(t if len(shape) == 1 else t.view(shape))
         return out
 
 
@@ -143,23 +146,11 @@ _TORCH_DTYPE = {np.dtype(np.int64): torch.int64, np.dtype(np.int32): torch.int32
 
 
 def _runs(first: np.ndarray, count: np.ndarray, out: np.ndarray | None = None) -> np.ndarray:
-    """Concatenation over i of first[i], first[i] + 1, ..., first[i] + count[i] - 1 (int64; count >= 0), computed as
-    one cumulative sum: a step array of ones whose entry at each run's start holds the jump from the previous run's
-    last value (from 0 for the first run)."""
-    total = int(count.sum())
-    steps = np.ones(total, dtype=np.int64) if out is None else out
-    if out is not None:
-        steps[:] = 1
-    keep = count > 0
-    f, c = first[keep], count[keep]
-    if f.size:
-        starts = np.cumsum(c) - c
-        prev_last = np.empty_like(f)
-        prev_last[0] = 0
-        prev_last[1:] = f[:-1] + c[:-1] - 1
-        steps[starts] = f - prev_last
-        np.cumsum(steps, out=steps)
-    return steps
+    """Concatenation over i of first[i], first[i] + 1, ..., first[i] + count[i] - 1 (int64; count >= 0): each run's
+    first value less where the run starts, repeated over the run, plus the places 0, 1, 2, ..."""
+    ends = np.cumsum(count)
+    shift = np.repeat(first - (ends - count), count)
+    return np.add(shift, np.arange(shift.size), out=out)
 
 
 @dataclass
@@ -174,15 +165,12 @@ class _Batch:
 
     @classmethod
     def of(cls, seqs) -> "_Batch":
-        n = len(seqs)
-        cols = np.array([(s.seq_length, s.num_cached_tokens, len(s.block_table)) for s in seqs],
-                        dtype=np.int64).reshape(n, 3)
-        nblk = cols[:, 2].copy()
-        flat = np.fromiter((b for s in seqs for b in s.block_table), dtype=np.int64, count=int(nblk.sum()))
-        row_start = np.zeros(n, dtype=np.int64)
-        if n > 1:
-            np.cumsum(nblk[:-1], out=row_start[1:])
-        return cls(cols[:, 0].copy(), cols[:, 1].copy(), nblk, flat, row_start)
+        tables = [s.block_table for s in seqs]
+        nblk = np.array([len(t) for t in tables], dtype=np.int64)
+        flat = np.array(list(chain.from_iterable(tables)), dtype=np.int64)
+        row_start = np.cumsum(nblk) - nblk
+        return cls(np.array([s.seq_length for s in seqs], dtype=np.int64),
+                   np.array([s.num_cached_tokens for s in seqs], dtype=np.int64), nblk, flat, row_start)
 
     def padded_tables(self, out: np.ndarray) -> None:
         """Writes the -1 padded [n, width] tables into ``out`` (rows in order, entries in order)."""
@@ -198,9 +186,15 @@ def prefill_slots(batch: _Batch, block_size: int) -> np.ndarray:
     consecutive, so each (sequence, block) piece is one run starting at table[block] * bs + first token % bs."""
     bs = block_size
     q = batch.length - batch.cached
+    first_blk = batch.cached // bs
+    pieces = (batch.length - 1) // bs - first_blk + 1
     live = (q > 0) & (batch.nblk > 0)
-    first_blk = np.where(live, batch.cached // bs, 0)
-    pieces = np.where(live, (batch.length - 1) // bs - first_blk + 1, 0)
+    if live.all():
+        if (pieces == 1).all():  # every sequence's tokens lie in one block, one run each: short prompts, decode-like steps
+            return _runs((batch.flat[batch.row_start + first_blk] - first_blk) * bs + batch.cached, q)
+    else:
+        first_blk = np.where(live, first_blk, 0)
+        pieces = np.where(live, pieces, 0)
     col = _runs(first_blk, pieces)                                      # table column of each piece
     entry = batch.flat[_runs(batch.row_start + first_blk, pieces)]      # its block id
     lo = np.maximum(np.repeat(batch.cached, pieces), col * bs)          # first token of the piece
@@ -216,19 +210,19 @@ def prepare_prefill_context(seqs, block_size: int, device="cuda", graphs: bool =
     batch = _Batch.of(seqs)
     n = len(seqs)
     q = batch.length - batch.cached
-    total_q = int(q.sum())
+    ends_q = np.cumsum(q)
+    total_q = int(ends_q[-1]) if n else 0
     with_tables = graphs or bool((batch.cached > 0).any())
     slots = prefill_slots(batch, block_size)
-    width = int(batch.nblk.max(initial=0))
     stage = staging or StepStaging(device)
     specs = [(np.int64, (total_q,)), (np.int32, (n + 1,)), (np.int32, (n + 1,)), (np.int32, (slots.size,))]
     if with_tables:
-        specs.append((np.int32, (n, width)))
+        specs.append((np.int32, (n, int(batch.nblk.max(initial=0)))))
     views = stage.layout(specs)
-    _runs(batch.cached, q, out=views[0])
-    for cu, lens in ((views[1], q), (views[2], batch.length)):
-        cu[0] = 0
-        np.cumsum(lens, out=cu[1:])
+    np.add(np.repeat(batch.cached - (ends_q - q), q), np.arange(total_q), out=views[0])  # _runs(cached, q)
+    views[1][0] = views[2][0] = 0
+    views[1][1:] = ends_q
+    np.cumsum(batch.length, out=views[2][1:])
     views[3][:] = slots
     if with_tables:
         batch.padded_tables(views[4])

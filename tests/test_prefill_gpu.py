@@ -781,3 +781,79 @@ def test_mixed_step_with_the_riding_store_replays_in_a_hip_graph():
         assert torch.equal(layer.k_cache, kc_want) and torch.equal(layer.v_cache, vc_want)
     finally:
         reset_context()
+
+
+@pytest.mark.parametrize("pre,prefix,bs", [
+    ([192], [0], 256), ([193, 1, 64], [0, 0, 0], 64), ([200, 5], [1, 63], 256), ([256], [64], 64), ([257, 130], [65, 200], 256),
+    ([1] * 40 + [30] * 60, [0] * 50 + [33] * 50, 256), ([9] * 300, [47, 48, 49] * 100, 64), ([100] * 40, [31] * 40, 256)],
+    ids=["192", "193", "prefix 1", "prefix 64", "prefix 65", "100 short", "300 x 9", "40 x 100"])
+def test_items_of_32_row_blocks(pre, prefix, bs):
+    """64-row items as two row blocks x two key halves (from 192 tokens on) and 128-row items as four row blocks (large
+    grids): one key tile and several, both parities of the tile count, tiles with one key, halves without keys, the first
+    new key inside, at and past a tile's edge. The riding store against store then attend (bit-identical outputs and
+    caches), and both against the oracle; packed keys too where nothing is cached."""
+    from voxcpm2_arabic_dialects_turbo_amd.ops import prefill_attention_store, varlen_attention
+
+    gen = torch.Generator().manual_seed(120 + len(pre) + pre[0])
+    nq, nk, kc, vc, tables, q, k, v, slots = _step_with_new_rows(gen, pre, prefix, [], HK, bs)
+    cu_q, cu_k, bt, sl = _cu(nq).to(DEV), _cu(nk).to(DEV), tables.to(DEV), slots.to(DEV)
+    kc1, vc1 = kc.to(DEV), vc.to(DEV)
+    kc2, vc2 = kc1.clone(), vc1.clone()
+    fused = prefill_attention_store(q, k, v, kc1, vc1, sl, cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=max(nq),
+                                    softmax_scale=SCALE, block_table=bt)
+    store_kvcache(k, v, kc2, vc2, sl)
+    two = varlen_attention(q, None, None, cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=max(nq), softmax_scale=SCALE,
+                           causal=True, block_table=bt, k_cache=kc2, v_cache=vc2)
+    torch.cuda.synchronize()
+    assert torch.equal(fused, two) and torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
+    want = ref.varlen(q.float().cpu(), _cu(nq), _cu(nk), k_cache=kc2.cpu(), v_cache=vc2.cpu(), block_tables=tables)
+    attn_close(fused, want, "paged")
+    if not any(prefix):
+        out = flash_attn_varlen_func(q, k, v, cu_q, cu_q, max(nq), max(nq), softmax_scale=SCALE, causal=True)
+        attn_close(out, want, "packed")
+
+
+@pytest.mark.parametrize("h,hk,n", [(64, 2, 40), (64, 1, 20), (128, 1, 130), (2, 2, 2000), (8, 4, 500), (16, 2, 333)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_group_sizes_over_32_row_blocks(h, hk, n, causal):
+    """Group sizes 1 to 128 in the 64-row and 128-row items of 32-row blocks, causal and not."""
+    gen = torch.Generator().manual_seed(140 + h + hk)
+    lens = [n, n // 2 + 1]
+    q, k, v = randn(gen, sum(lens), h, D), randn(gen, sum(lens), hk, D), randn(gen, sum(lens), hk, D)
+    cu = _cu(lens)
+    out = flash_attn_varlen_func(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), cu.to(DEV), n, n, softmax_scale=SCALE,
+                                 causal=causal)
+    attn_close(out, ref.varlen(q.float(), cu, cu, k=k, v=v, causal=causal), f"{h}/{hk} heads, {n} tokens")
+
+
+def test_query_rows_past_a_descriptors_offsets():
+    """Query rows 2^23 elements apart take per-lane addresses instead of a buffer descriptor: the same output bits."""
+    gen = torch.Generator().manual_seed(150)
+    L, step = 192, 1 << 23
+    q, k, v = randn(gen, L, H, D).to(DEV), randn(gen, L, HK, D).to(DEV), randn(gen, L, HK, D).to(DEV)
+    far = torch.empty((L - 1) * step + H * D, dtype=torch.bfloat16, device=DEV).as_strided((L, H, D), (step, D, 1))
+    far.copy_(q)
+    cu = _cu([L]).to(DEV)
+    kw = dict(softmax_scale=SCALE, causal=True)
+    assert torch.equal(flash_attn_varlen_func(far, k, v, cu, cu, L, L, **kw),
+                       flash_attn_varlen_func(q, k, v, cu, cu, L, L, **kw))
+
+
+@pytest.mark.parametrize("lens", [[260, 33], [90] * 90], ids=["64-row items", "128-row items"])
+def test_unmapped_blocks_in_items_of_32_row_blocks(lens):
+    """An unmapped first block (NaN in the slots a wrong read would meet) takes no weight, nor does a whole unmapped
+    context: the oracle over the keys that are left."""
+    gen = torch.Generator().manual_seed(160 + len(lens))
+    nk = [n + 128 for n in lens]
+    kc, vc, tables = paged_pool(gen, nk, sum(-(-n // 64) for n in nk) + 2, block_size=64)
+    t_gpu = tables.clone()
+    t_gpu[:, 0] = -1
+    t_gpu[1, :] = 10 ** 6
+    kc[tables[:, 0].long()] = float("nan")
+    vc[tables[:, 0].long()] = float("nan")
+    q = randn(gen, sum(lens), H, D)
+    out = flash_attn_varlen_func(q.to(DEV), kc.to(DEV), vc.to(DEV), _cu(lens).to(DEV), _cu(nk).to(DEV), max(lens), max(nk),
+                                 softmax_scale=SCALE, causal=True, block_table=t_gpu.to(DEV))
+    want = ref.varlen(q.float(), _cu(lens), _cu([n - 64 for n in nk]), k_cache=kc, v_cache=vc, block_tables=tables[:, 1:])
+    want[lens[0]:lens[0] + lens[1]] = 0
+    attn_close(out, want, "unmapped")

@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "decode_body.h"
+#include "prefill_tile32.h"
 #include "vox_common.h"
 #include "vox_kernels.h"
 
@@ -52,10 +53,15 @@ constexpr int kVsStride = kD + 24;
 constexpr int kBufferWord3 = 0x00020000;
 constexpr unsigned kXcds = 8;                  // MI355X: workgroups are dealt round-robin over 8 XCDs
 constexpr unsigned kXcdOrderMinWorkgroups = 1024;
-// Grids of up to this many workgroups take 8-wave workgroups (measured, bf16 output, causal: 1 x 512 tokens 14.5 ->
-// 12.2 us, 44 x 46 paged over a 50-token prefix -4 %, 16 x 512 -3 %, 4 x 2048 -4 %, 2 x 8192 -3 %; at 4096
-// workgroups (16 x 2048, 64 x 512) the 4-wave form is 2-3 % faster).
+// Paged caches of other block sizes: 128-row grids of up to this many workgroups take 8-wave workgroups (half of a wave's
+// work per key tile), larger ones 4 waves of 32 rows (fewer LDS reads per MFMA).
 constexpr int64_t kSmallGridWorkgroups = 2048;
+// 64-row items of sequences of at least this many of them (192 tokens at 8 heads per kv head) run as two row blocks x two
+// key halves (prefill_tile32.h), where a wave's work per key tile is halved; on fewer the merge of the halves costs more
+// than that saves. Packed, 16-row waves against key halves: 1 x 130 tokens 6.3 -> 6.7 us, 1 x 237 8.5 -> 7.9, 4 x 250-300
+// 11.4 -> 10.6, 1 x 1000 19.4 -> 15.9; paged with the store riding 1 x 64 5.2 -> 6.0, 1 x 237 8.9 -> 8.7. (Beyond two
+// workgroups per CU, in the rank-major order, the 16-row waves stay: 8 x 64-512 16.1 -> 16.6 us.)
+constexpr int64_t kSplitMinTiles = 24;
 // Grid forms of prefill_kernel (below)
 constexpr int kFormGrid = 0;
 constexpr int kFormPersistent = 1;
@@ -1008,6 +1014,23 @@ __device__ __forceinline__ void store_rows(const PrefillArgs& p, int wid) {
   }
 }
 
+// The plain grid's work item of this workgroup (with xcd_order, its XCD's next one)
+__device__ __forceinline__ void grid_item(const PrefillArgs& p, int& qt, int& b, int& g) {
+  qt = blockIdx.x;
+  b = blockIdx.y;
+  g = blockIdx.z;
+  if (p.xcd_order) {
+    const unsigned nwg = gridDim.x * gridDim.y * gridDim.z;
+    const unsigned id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const unsigned xq = nwg / kXcds, xr = nwg % kXcds, xcd = id % kXcds, loc = id / kXcds;
+    const unsigned work = (xcd < xr ? xcd * (xq + 1) : xr * (xq + 1) + (xcd - xr) * xq) + loc;
+    qt = (int)(work % gridDim.x);
+    b = (int)((work / gridDim.x) % gridDim.y);
+    g = (int)(work / (gridDim.x * gridDim.y));
+    if (p.causal) qt = (int)gridDim.x - 1 - qt;  // heavy query tiles first
+  }
+}
+
 // Waves per SIMD the registers must allow: two 4-wave workgroups per CU (their 64 KB of LDS each fits twice), two
 // 8-wave ones (at most 128 VGPRs: the riding store's paged form would take 132 and hold one workgroup per CU, which
 // ran the 44 x 46-token step's 264 workgroups in two rounds, 15.4 -> 17.6 us), one int8 workgroup (128 KB of LDS).
@@ -1035,22 +1058,54 @@ __global__ __launch_bounds__(64 * NW * (QUANT ? 2 : 1), prefill_waves_per_simd(Q
     prefill_items<QUANT, KV, NW, RT>(p, (int)blockIdx.x, (int)gridDim.x, bufs,
                                      item_lds(s_items, kMaxSeqPerLaunch, NWV));
   } else {
-    int qt = blockIdx.x, b = blockIdx.y, gz = blockIdx.z;
-    if (p.xcd_order) {
-      const unsigned nwg = gridDim.x * gridDim.y * gridDim.z;
-      const unsigned id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-      const unsigned xq = nwg / kXcds, xr = nwg % kXcds, xcd = id % kXcds, loc = id / kXcds;
-      const unsigned work = (xcd < xr ? xcd * (xq + 1) : xr * (xq + 1) + (xcd - xr) * xq) + loc;
-      qt = (int)(work % gridDim.x);
-      b = (int)((work / gridDim.x) % gridDim.y);
-      gz = (int)(work / (gridDim.x * gridDim.y));
-      if (p.causal) qt = (int)gridDim.x - 1 - qt;  // heavy query tiles first
-    }
+    int qt, b, gz;
+    grid_item(p, qt, b, gz);
     prefill_tile<QUANT, KV, NW, RT>(p, qt, b, gz, bufs);
     if constexpr (KV == kPacked || KV == kPagedTilesRows) {
       if (p.store_rows > 0) {
         const int id = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
         if (id >= p.store_first && id < p.store_first + p.store_wgs) store_rows(p, id - p.store_first);
+      }
+    }
+  }
+}
+
+// The bf16 kernel over packed keys or paged tiles (prefill_tile32.h), in the plain grid. 4 waves, two workgroups per CU
+// (64 KB of LDS and at most 256 VGPRs each).
+template <int SRC, int RG, int KS>
+__global__ __launch_bounds__(64 * RG * KS, 2) void prefill32_kernel(PrefillArgs p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t kt0[kTB];
+  __shared__ __attribute__((aligned(1024))) uint8_t kt1[kTB];
+  __shared__ __attribute__((aligned(1024))) uint8_t vt0[kTB];
+  __shared__ __attribute__((aligned(1024))) uint8_t vt1[kTB];
+  __shared__ float red[KS == 2 ? 128 : 1];
+  const pf32::Bufs bufs{kt0, kt1, vt0, vt1, red};
+  int qt, b, g;
+  grid_item(p, qt, b, g);
+  pf32::tile<SRC, RG, KS>(p, qt, b, g, bufs);
+  if constexpr (SRC != pf32::kCache) {
+    // the riding store; its arguments read here, not held in scalar registers through the item
+    typedef const __attribute__((address_space(4))) PrefillArgs* KernArgs;
+    KernArgs late = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(late));
+    if (late->store_rows > 0) {
+      const int wid = late->store_light > 0
+                          ? (qt < late->store_light ? qt + late->store_light * (b + late->batch * g) : INT32_MAX)
+                          : (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)) - late->store_first;
+      if (wid >= 0 && wid < late->store_wgs) {
+        PrefillArgs a{};
+        a.num_kv_heads = late->num_kv_heads;
+        a.k_src = late->k_src;
+        a.v_src = late->v_src;
+        a.k_row_stride = late->k_row_stride;
+        a.v_row_stride = late->v_row_stride;
+        a.store_slots = late->store_slots;
+        a.store_k_cache = late->store_k_cache;
+        a.store_v_cache = late->store_v_cache;
+        a.store_rows = late->store_rows;
+        a.store_num_slots = late->store_num_slots;
+        a.store_wgs = late->store_wgs;
+        store_rows(a, wid);
       }
     }
   }
@@ -1105,17 +1160,36 @@ static int device_cus() {
 template <bool QUANT, int NW, int RT, int FORM = kFormGrid>
 hipError_t launch_prefill_kind(const PrefillArgs& a, dim3 grid, hipStream_t stream) {
   const dim3 block(64 * NW * (QUANT ? a.num_kv_heads : 1));
-  if (!a.block_tables)
+  if (a.block_tables && a.block_size % kBK) {
+    if (a.new_from_rows) return hipErrorInvalidValue;
+    prefill_kernel<QUANT, kPagedPieces, NW, RT, FORM><<<grid, block, 0, stream>>>(a);
+  } else if constexpr (!QUANT && NW * RT != 4) {
+    return hipErrorInvalidValue;  // bf16 items of 128 rows over keys in tiles: launch_prefill32
+  } else if (!a.block_tables) {
     prefill_kernel<QUANT, kPacked, NW, RT, FORM><<<grid, block, 0, stream>>>(a);
-  else if (a.block_size % kBK == 0 && a.new_from_rows) {
+  } else if (a.new_from_rows) {
     if constexpr (FORM != kFormPersistent)  // (the plain and rank-major forms take a riding store)
       prefill_kernel<QUANT, kPagedTilesRows, NW, RT, FORM><<<grid, block, 0, stream>>>(a);
     else
       return hipErrorInvalidValue;
-  } else if (a.block_size % kBK == 0)
+  } else {
     prefill_kernel<QUANT, kPagedTiles, NW, RT, FORM><<<grid, block, 0, stream>>>(a);
+  }
+  return hipGetLastError();
+}
+
+// Keys in 64-key tiles (packed, or paged blocks that are a multiple of 64): the forms of prefill32_kernel
+bool tiled_keys(const PrefillArgs& a) { return !a.block_tables || a.block_size % kBK == 0; }
+template <int RG, int KS>
+hipError_t launch_prefill32(const PrefillArgs& a, dim3 grid, hipStream_t stream) {
+  if (!tiled_keys(a) || (32 * RG) % a.group) return hipErrorInvalidValue;
+  const dim3 block(64 * RG * KS);
+  if (!a.block_tables)
+    prefill32_kernel<pf32::kRows, RG, KS><<<grid, block, 0, stream>>>(a);
+  else if (a.new_from_rows)
+    prefill32_kernel<pf32::kCacheNew, RG, KS><<<grid, block, 0, stream>>>(a);
   else
-    prefill_kernel<QUANT, kPagedPieces, NW, RT, FORM><<<grid, block, 0, stream>>>(a);
+    prefill32_kernel<pf32::kCache, RG, KS><<<grid, block, 0, stream>>>(a);
   return hipGetLastError();
 }
 
@@ -1190,6 +1264,15 @@ hipError_t launch_prefill(const PrefillArgs& a0, int max_seqlen_q, hipStream_t s
   auto store_by = [&](int64_t nwg) {
     a.store_wgs = a.store_rows > 0 ? (int)(nwg < 256 ? nwg : 256) : 0;
     a.store_first = (int)(nwg - a.store_wgs < 256 ? nwg - a.store_wgs : 256);
+    a.store_light = 0;
+  };
+  // ... in a plain causal grid over paged tiles or packed keys by the workgroups of each sequence's first half of the q
+  // tiles, the ones with the short chains (one prompt of 237 tokens: the copy behind the longest chain cost 0.7 us)
+  auto store_by_light = [&](int64_t q_tiles) {
+    if (a.store_rows <= 0 || !a.causal || a.xcd_order || q_tiles < 8 || (a.block_tables && a.block_size % kBK)) return;
+    a.store_light = (int)((q_tiles + 1) / 2);
+    const int64_t wgs = a.store_light * (int64_t)a.batch * a.num_kv_heads;
+    a.store_wgs = (int)(wgs < 256 ? wgs : 256);
   };
   const bool fits64 = 64 % a.group == 0;  // group sizes above 64 take the 128-row form only
   const int64_t tiles64 = fits64 ? (max_seqlen_q + 64 / a.group - 1) / (64 / a.group) : 0;
@@ -1199,6 +1282,10 @@ hipError_t launch_prefill(const PrefillArgs& a0, int max_seqlen_q, hipStream_t s
     store_by(grid64);
     if (a.causal && grid64 > 2 * cus && grid64 <= INT32_MAX)
       return launch_prefill_kind<false, 4, 1, kFormRanked>(a, dim3((unsigned)grid64), stream);
+    if (tiled_keys(a) && tiles64 >= kSplitMinTiles) {
+      store_by_light(tiles64);
+      return launch_prefill32<2, 2>(a, dim3((unsigned)tiles64, (unsigned)a.batch, (unsigned)a.num_kv_heads), stream);
+    }
     return launch_prefill_kind<false, 4, 1>(a, dim3((unsigned)tiles64, (unsigned)a.batch, (unsigned)a.num_kv_heads),
                                             stream);
   }
@@ -1208,6 +1295,10 @@ hipError_t launch_prefill(const PrefillArgs& a0, int max_seqlen_q, hipStream_t s
   a.xcd_order = nwg >= kXcdOrderMinWorkgroups;
   store_by(nwg);
   const dim3 grid((unsigned)q_tiles, (unsigned)a.batch, (unsigned)a.num_kv_heads);
+  if (tiled_keys(a)) {
+    store_by_light(q_tiles);
+    return launch_prefill32<4, 1>(a, grid, stream);
+  }
   if (nwg <= kSmallGridWorkgroups) return launch_prefill_kind<false, 8, 1>(a, grid, stream);
   return launch_prefill_kind<false, 4, 2>(a, grid, stream);
 }

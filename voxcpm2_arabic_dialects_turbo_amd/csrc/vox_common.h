@@ -12,6 +12,7 @@ namespace vox {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -24,6 +25,14 @@ constexpr float kLog2e = 1.4426950408889634f;
 // agree, which the kernels use to feed operands straight from memory.
 __device__ __forceinline__ f32x4 mfma_16x16x32(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                 0, 0, 0);
+}
+
+// D(32x32 fp32) += A(32x16 bf16) * B(16x32 bf16).
+// Lane l holds A[row = l%32][k = 8*(l/32) .. +8), B[k = 8*(l/32) .. +8)[col = l%32] and, in register i,
+// D[row = 8*(i/4) + 4*(l/32) + i%4][col = l%32].
+__device__ __forceinline__ f32x16 mfma_32x32x16(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
                                                  0, 0, 0);
 }
 

@@ -114,6 +114,7 @@ struct PrefillArgs {
   int64_t store_num_slots;
   int store_first;
   int store_wgs;
+  int store_light;            // > 0: instead by the workgroups of q tiles below it, numbered q tile first, then sequence
   // paged keys with the step's new keys in rows (launch_mixed with a riding store): sequence b's keys at positions
   // nk - nq and later (its nq new tokens, stored by this launch's merge kernel) come from k_src / v_src rows
   // cu_q[b] + (position - (nk - nq)) instead of the cache; the earlier keys through the block table as usual

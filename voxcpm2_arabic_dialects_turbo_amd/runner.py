@@ -120,7 +120,8 @@ class StepStaging:
         if dev.type == "cuda":
             dst = src.to(dev, non_blocking=True)
             if self._slot is not None:
-                if self._slot.done is None:
+                # (an event belongs to the device it was first recorded on: device "cuda" follows the current one)
+                if self._slot.done is None or self._slot.done.device != dst.device:
                     self._slot.done = torch.cuda.Event()
                 self._slot.done.record()
                 self._slot.pending = True

@@ -153,9 +153,9 @@ size_t vox_prefill_workspace_bytes(int batch);
  * vox_prefill_attn over the packed rows key / value (no block table) (reference: the prefill branch of
  * nanovllm_voxcpm/model/layers.py:326-348 without a block table, store_kvcache then flash_attn_varlen_func over the
  * step's own k and v). The attention reads the packed rows, not the cache, so the copy rides in the attention launch
- * (the last workgroups copy the rows after their own work) instead of a launch of its own. Outputs and caches are
- * identical to the two calls. Rows the 16-byte copy cannot move (16-byte aligned rows, strides multiples of 8) take
- * the two calls. Arguments as in those two functions; num_tokens = the rows of key / value and slot_mapping. */
+ * (workgroups that have done their own work, or have none, copy the rows) instead of a launch of its own. Outputs and
+ * caches are identical to the two calls. Rows the 16-byte copy cannot move (16-byte aligned rows, strides multiples of
+ * 8) take the two calls. Arguments as in those two functions; num_tokens = the rows of key / value and slot_mapping. */
 int vox_prefill_attn_store(const void* q, int64_t q_row_stride, const void* key, const void* value,
                            int64_t key_row_stride, int64_t value_row_stride, const int32_t* slot_mapping,
                            void* k_cache, void* v_cache, int64_t num_slots, int64_t num_tokens,
@@ -171,9 +171,9 @@ int vox_prefill_attn_store(const void* q, int64_t q_row_stride, const void* key,
  * With blocks of a multiple of 64 tokens and rows 16-byte aligned with strides multiples of 8 (below 2^24 elements),
  * the store rides in the attention launch: each sequence's new keys (its last nq key positions) are read from the
  * rows key / value (row cu_seqlens_q[b] + i for the i-th) instead of the cache, and the rows are written into the
- * caches after the reads: by the merge kernel when the call runs as one mixed launch (vox_prefill_attn's conditions:
+ * caches: after the reads by the merge kernel when the call runs as one mixed launch (vox_prefill_attn's conditions:
  * workspace, up to 256 sequences, some sequence with more than one query), else, when it runs on the prefill kernel
- * alone (no workspace), by the launch's last workgroups. That equals the two calls when, as the engine's scheduler
+ * alone (no workspace), beside the reads by workgroups of the launch. That equals the two calls when, as the engine's scheduler
  * guarantees, slot_mapping holds for each sequence's new tokens the slots its block table gives their positions, and
  * no sequence's new slots lie inside another sequence's context. Otherwise (a workspace whose call is not one mixed
  * launch, other block sizes, other rows) the two calls run. Outputs and caches are identical to the two calls;

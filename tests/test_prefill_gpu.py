@@ -813,6 +813,33 @@ def test_items_of_32_row_blocks(pre, prefix, bs):
         attn_close(out, want, "packed")
 
 
+@pytest.mark.parametrize("n_seq,n", [(1, 1), (1, 37), (227, 8), (228, 8), (255, 8), (256, 8), (15, 136), (44, 50), (62, 60),
+                                     (1, 1000), (1, 2048)])
+@pytest.mark.parametrize("hk", [1, 2])
+def test_riding_store_copied_beside_the_items(n_seq, n, hk):
+    """Plain grids with room for copying workgroups beside their items (two workgroups per CU) and without: one workgroup,
+    as many rows a copying workgroup as the rule allows and one more (227 and 228 sequences of 8 tokens on 256 CUs), grids
+    one item short of full and full, 128-row items, one long sequence. Paged keys with prefixes and packed keys: outputs
+    and caches bit-identical to store then attend."""
+    from voxcpm2_arabic_dialects_turbo_amd.ops import prefill_attention_store
+
+    gen = torch.Generator().manual_seed(140 + n_seq + n)
+    nq, nk, kc, vc, tables, q, k, v, slots = _step_with_new_rows(gen, [n] * n_seq, [(5 * i) % 70 for i in range(n_seq)], [],
+                                                                 hk, 64)
+    cu_q, cu_k, bt, sl = _cu(nq).to(DEV), _cu(nk).to(DEV), tables.to(DEV), slots.to(DEV)
+    kc2, vc2 = kc.to(DEV), vc.to(DEV)
+    kc1, vc1, kc0, vc0 = kc2.clone(), vc2.clone(), kc2.clone(), vc2.clone()
+    kw = dict(cu_seqlens_q=cu_q, max_seqlen_q=n, softmax_scale=SCALE)
+    paged = prefill_attention_store(q, k, v, kc1, vc1, sl, cu_seqlens_k=cu_k, block_table=bt, **kw)
+    packed = prefill_attention_store(q, k, v, kc0, vc0, sl, cu_seqlens_k=cu_q, **kw)
+    store_kvcache(k, v, kc2, vc2, sl)
+    want = flash_attn_varlen_func(q, kc2, vc2, cu_q, cu_k, n, max(nk), softmax_scale=SCALE, causal=True, block_table=bt)
+    want_packed = flash_attn_varlen_func(q, k, v, cu_q, cu_q, n, n, softmax_scale=SCALE, causal=True)
+    torch.cuda.synchronize()
+    assert torch.equal(paged, want) and torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
+    assert torch.equal(packed, want_packed) and torch.equal(kc0, kc2) and torch.equal(vc0, vc2)
+
+
 @pytest.mark.parametrize("h,hk,n", [(64, 2, 40), (64, 1, 20), (128, 1, 130), (2, 2, 2000), (8, 4, 500), (16, 2, 333)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_group_sizes_over_32_row_blocks(h, hk, n, causal):

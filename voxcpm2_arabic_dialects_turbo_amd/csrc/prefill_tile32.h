@@ -75,7 +75,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
   asm volatile("" ::"s"(p.q), "s"(p.q_row_stride), "s"(p.out), "s"(p.out_row_stride), "s"(p.cu_q), "s"(p.cu_k),
                "s"(p.group), "s"(p.causal), "s"(p.scale_log2), "s"(p.row_limit), "s"(p.skip_single));
   if constexpr (SRC != kCache)
-    asm volatile("" ::"s"(p.k_src), "s"(p.v_src), "s"(p.k_row_stride), "s"(p.v_row_stride));
+    asm volatile("" ::"s"(p.k_src), "s"(p.v_src), "s"(p.k_row_stride), "s"(p.v_row_stride), "s"(p.num_kv_heads));
   if constexpr (SRC != kRows)
     asm volatile("" ::"s"(p.block_tables), "s"(p.bt_stride), "s"(p.max_blocks), "s"(p.block_size), "s"(p.num_blocks),
                  "s"(p.k_cache), "s"(p.v_cache), "s"(p.num_kv_heads));
@@ -100,6 +100,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
   const int gsh = __builtin_ctz(p.group);  // the group divides 128: a power of two
   const int BQ = ROWS >> gsh;              // query tokens of the item
   if (qt * BQ >= nq || (p.skip_single && nq == 1)) return;  // (one-query rows: the decode kernel's, in varlen mode)
+  if (SRC != kCache && g >= p.num_kv_heads) return;         // a workgroup that only copies (a riding store)
 
   // ---- this lane's query row
   const int rho = rg * 32 + col;

@@ -106,7 +106,7 @@ struct PrefillArgs {
   // KV store riding in a packed launch (vox_prefill_attn_store): rows i < store_rows of k_src / v_src go to cache slot
   // store_slots[i] of store_k_cache / store_v_cache (rows of num_kv_heads * 128; -1 and slots outside
   // [0, store_num_slots) skipped), copied by workgroups [store_first, store_first + store_wgs) (launch order) after
-  // their work item
+  // their work item; from the item count on, workgroups without one (a plane of the grid past the kv heads)
   const int32_t* store_slots;
   uint16_t* store_k_cache;
   uint16_t* store_v_cache;

@@ -144,6 +144,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, int qt, int b
   const int G = p.group;
   const int BQ = ROWS / G;  // query tokens per workgroup
   if (qt * BQ >= nq || (p.skip_single && nq == 1)) return;  // (one-query rows: the decode kernel's, in varlen mode)
+  if constexpr (!QUANT && (KV == kPacked || KV == kPagedTilesRows))
+    if (gz >= p.num_kv_heads) return;  // a workgroup that only copies (a riding store)
 
   const int tid = threadIdx.x & (NT - 1);  // thread within the half
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
@@ -1060,9 +1062,7 @@ __global__ __launch_bounds__(64 * NW * (QUANT ? 2 : 1), prefill_waves_per_simd(Q
   } else {
     int qt, b, gz;
     grid_item(p, qt, b, gz);
-    // (workgroups past the kv heads' planes only copy: store_beside in launch_prefill)
-    if (QUANT || (KV != kPacked && KV != kPagedTilesRows) || blockIdx.z < (unsigned)p.num_kv_heads)
-      prefill_tile<QUANT, KV, NW, RT>(p, qt, b, gz, bufs);
+    prefill_tile<QUANT, KV, NW, RT>(p, qt, b, gz, bufs);
     if constexpr (KV == kPacked || KV == kPagedTilesRows) {
       if (p.store_rows > 0) {
         const int id = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));

@@ -13,7 +13,7 @@ from oracle import attention as ref
 from tests._util import BLOCK, D, H, HK, attn_close, paged_pool, randn, uniform_lens
 from tests.golden import make_golden
 from voxcpm2_arabic_dialects_turbo_amd import _lib
-from voxcpm2_arabic_dialects_turbo_amd.ops import decode_attention, flash_attn_with_kvcache
+from voxcpm2_arabic_dialects_turbo_amd.ops import decode_attention, decode_workspace, flash_attn_with_kvcache
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -171,6 +171,26 @@ def test_decode_merge_forms(lens):
     for i, n in enumerate(lens):
         if n == 0:
             assert int(out[i].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("lens,ranges", [
+    ([40] * 150, 150), ([64] * 30 + [0] * 40 + [49] * 31, 61), ([16] * 3, 3), ([0, 0, 33, 0, 48], 2), ([20] + [64] * 8, 34),
+    ([10, 30] * 50, 150), ([100], 7), ([420], 27), ([480], 30), ([800], 30), ([2048], 32), ([65] * 70, 350), ([1] * 300, 300)],
+    ids=["150x40", "61x4 steps, empty rows", "3x1 step", "2x3 steps, empty rows", "one shorter", "100x1-2 steps", "100",
+         "420", "480", "800", "2048", "70x5 steps", "300x1"])
+def test_decode_ranges_of_short_and_long_steps(lens, ranges):
+    """How many ranges a launch cuts its 16-token steps into: a range a sequence where all are equally long and at most
+    four steps (a wave each), ranges of one step up to 30 a sequence, of up to four beyond; never more than the
+    workgroups. The active count is what the split kernel left behind the step layout in the workspace."""
+    gen = torch.Generator().manual_seed(170 + len(lens) + lens[0])
+    kc, vc, tables = paged_pool(gen, [max(n, 1) for n in lens], sum(-(-max(n, 1) // BLOCK) for n in lens) + 2)
+    (_, _), out = _check(randn(gen, len(lens), H, D), kc, vc, lens, tables, f"{len(lens)} sequences")
+    assert not out[torch.tensor([n == 0 for n in lens], device=out.device)].any()
+    grid = _lib.load().vox_decode_workgroups()
+    partials = -(-(len(lens) + grid) * (16 * D + 32) * 4 // 256) * 64  # (the layout's place, in 4-byte words)
+    layout = decode_workspace(out.device).view(torch.int32)[partials:partials + len(lens) + 2].tolist()
+    assert layout[-2] == sum(-(-n // 16) for n in lens)
+    assert layout[-1] == min(ranges, grid)
 
 
 def test_decode_repeated_calls_of_changing_batch():

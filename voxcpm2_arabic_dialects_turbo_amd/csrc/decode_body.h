@@ -58,11 +58,8 @@ constexpr int kMaxHeads = 16;
 #ifndef VOX_MERGE_BATCH
 #define VOX_MERGE_BATCH 8
 #endif
-// Most partials one sequence is cut into. A sequence of n steps meets at most about n G / S + 2 of G equal ranges of
-// S steps, so a launch uses G' = min(grid, S / 4, (kMaxPieces - 2) S / n_max) workgroups (the others leave after the layout
-// scan): a long sequence among few is not cut into one-step pieces, each a partial for the merge kernel to load.
-// Batches whose merge has four workgroups per sequence take twice the pieces (one stream of 4000 tokens: 13.7 us a layer
-// with 32, 12.9 with 64).
+// Pieces one sequence is cut into, at most: a sequence of n steps meets about n G / S + 2 of G equal ranges of S steps
+// (active_workgroups).
 constexpr int kMaxPieces = 32;
 constexpr int kMaxPiecesSplit = 64;
 // Batches of up to this many sequences merge with four workgroups per sequence (merge_row<4>), a quarter of the partials
@@ -148,13 +145,28 @@ __device__ __forceinline__ int64_t muldiv(int64_t a, int64_t b, int64_t c, int64
   return (int64_t)(num / (uint64_t)d);
 }
 
-// G' of a launch over `steps` steps whose longest sequence has `max_seq_steps`: at most one workgroup per kWaves steps (a
-// range of fewer leaves waves idle, takes as long, and adds a partial to merge: one stream of 420 tokens, 27 ranges of a
-// step each take 12.0 us a layer with their merge, 7 of four 10.0), so no range is empty
-__device__ __forceinline__ int active_workgroups(int grid, int64_t steps, int max_seq_steps, int batch) {
+// The workgroups G' <= grid a launch over `steps` steps uses, its longest sequence `max_seq_steps` long (the others leave
+// after the layout scan); no range is empty. us a layer of a step, 16-token steps:
+//  * Every sequence n <= kWaves steps long (or empty): a range each, so none is cut and none merged, and its n steps run
+//    on n waves at once (150 of 40 tokens: 9.5 us, 11.5 in ranges of one step, 11.8 in ranges of four; 150 of 64: 10.1,
+//    12.1, 10.0).
+//  * Else ranges of one step while no sequence is cut into more than kMaxPieces, whose partials the merge reads in one
+//    batch of loads a wave: a range of two to four steps wakes as many waves, but merges them in LDS first and, over
+//    short sequences, one segment after the other (ranges of one step against four: 1 of 420 tokens 9.0 and 10.1, 1 of
+//    100 8.2 and 9.3, 16 of 20-40 8.8 and 10.8, 150 of 8-16 8.1 and 11.2, 64 of 100 10.6 and 11.7).
+//  * Beyond, ranges grow with the longest sequence (two steps for one of 800 tokens: 9.4 us, 10.0 in ranges of four), with
+//    four merging workgroups per sequence only up to four steps, a step for each wave, and from there on again at
+//    kMaxPiecesSplit pieces (one stream of 4000 tokens: 13.7 us with 32 pieces, 12.9 with 64).
+__device__ __forceinline__ int active_workgroups(int grid, int64_t steps, int max_seq_steps, bool same, int batch) {
   if (max_seq_steps <= 0) return 1;
-  const int pieces = batch <= kMergeSplitBatch ? kMaxPiecesSplit : kMaxPieces;
-  const int64_t cap = min((steps + kWaves - 1) / kWaves, muldiv(pieces - 2, steps, 0, max_seq_steps));
+  int64_t cap;
+  if (same && max_seq_steps <= kWaves) {
+    cap = steps / max_seq_steps;
+  } else {
+    cap = min(steps, muldiv(kMaxPieces - 2, steps, 0, max_seq_steps));
+    if (batch <= kMergeSplitBatch)
+      cap = max(cap, min((steps + kWaves - 1) / kWaves, muldiv(kMaxPiecesSplit - 2, steps, 0, max_seq_steps)));
+  }
   return (int)max((int64_t)1, min((int64_t)grid, cap));
 }
 
@@ -454,7 +466,20 @@ __device__ __forceinline__ void decode_split(const DecodeArgs& p, const int g, c
     if (tid == 0) L.start[p.batch] = run;
     __syncthreads();
     S = uniform(run);
-    G = active_workgroups(grid, S, uniform(nmax), p.batch);
+    nmax = uniform(nmax);
+    bool same = false;  // every sequence that has steps has nmax of them (looked at where it matters)
+    if (nmax <= kWaves) {
+      bool other = false;
+      for (int bb = tid; bb < p.batch; bb += kThreads) {
+        const int n = L.start[bb + 1] - L.start[bb];
+        other = other || (n != 0 && n != nmax);
+      }
+      const uint64_t others = __builtin_amdgcn_ballot_w64(other);
+      if (lane == 0) L.wmax[w] = others != 0;
+      __syncthreads();
+      same = uniform(L.wmax[0] | L.wmax[1] | L.wmax[2] | L.wmax[3]) == 0;
+    }
+    G = active_workgroups(grid, S, nmax, same, p.batch);
     if (g == 0) {  // the layout decode_merge_kernel reads, then the active workgroup count (a record keeps it)
       for (int i = tid; i <= p.batch; i += kThreads) p.steps[i] = L.start[i];
       if (tid == 0) p.steps[p.batch + 1] = G;

@@ -884,3 +884,64 @@ def test_unmapped_blocks_in_items_of_32_row_blocks(lens):
     want = ref.varlen(q.float(), _cu(lens), _cu([n - 64 for n in nk]), k_cache=kc, v_cache=vc, block_tables=tables[:, 1:])
     want[lens[0]:lens[0] + lens[1]] = 0
     attn_close(out, want, "unmapped")
+
+
+def _with_high_keys(gen, lens, high, lean=0.3):
+    """q / k / v rows of sequences of these lengths whose queries lean along one direction per kv group, with the keys
+    ``high`` ({position: factor}, every sequence that has the position) along it: log2-scaled scores of about 16 factor."""
+    T = sum(lens)
+    u = torch.randn(HK, D, generator=gen)
+    q = (u.repeat_interleave(H // HK, dim=0).expand(T, H, D) + lean * torch.randn(T, H, D, generator=gen)).to(torch.bfloat16)
+    k, v, at = randn(gen, T, HK, D), randn(gen, T, HK, D), 0
+    for n in lens:
+        for pos, f in high.items():
+            if pos < n:
+                k[at + pos] = (u * f).to(torch.bfloat16)
+        at += n
+    return q, k, v
+
+
+_RISES = {"first tile": {5: 12.0}, "second tile": {64: 12.0}, "one key half": {70: 12.0}, "other half": {100: 12.0},
+          "both halves": {70: 9.0, 100: 14.0}, "last key": {10 ** 6: 0.0}, "every tile": {64 * i + 7 * i % 64: 5.0 * i for i in range(1, 40)},
+          "past bf16 of 2^127": {130: 60.0}, "falling": {3: 30.0, 90: 20.0, 200: 4.0}}
+
+
+@pytest.mark.parametrize("rise", list(_RISES))
+@pytest.mark.parametrize("lens", [[150], [300], [333, 192, 257], [300, 129] + [40] * 12, [64, 100, 250, 300, 410, 512, 80, 33]],
+                         ids=["16-row waves", "key halves", "3 of key halves", "128-row items", "rank order"])
+@pytest.mark.parametrize("form", ["packed", "paged", "riding", "prefix"])
+def test_scores_rising_past_the_first_tile(form, lens, rise):
+    """Keys whose scores pass the first tile's max by more than 62 log2 units, in each half of a tile, in the last tile,
+    in every tile, far beyond 2^127, and falling ones, over every bf16 form: the tiles of 16-row waves (redone with their
+    max) and of 32-row blocks (the row max raised ahead of the tile), from packed rows, cached keys, and new rows beside
+    cached ones (a riding store, with and without a prefix). Against the oracle; the cached forms bit for bit alike."""
+    from voxcpm2_arabic_dialects_turbo_amd.ops import prefill_attention_store
+
+    gen = torch.Generator().manual_seed(200 + len(lens))
+    prefix = 50 if form == "prefix" else 0
+    high = {max(lens) + prefix - 1: 12.0} if rise == "last key" else _RISES[rise]
+    full = [n + prefix for n in lens]
+    q, k, v = _with_high_keys(gen, full, high)
+    new = torch.cat([torch.arange(at - n, at) for n, at in zip(lens, np.cumsum(full).tolist())])  # rows of the new tokens
+    cu_q, cu_k = _cu(lens), _cu(full)
+    want = ref.varlen(q[new].float(), cu_q, cu_k, k=k, v=v)
+    kw = dict(cu_seqlens_q=cu_q.to(DEV), softmax_scale=SCALE, causal=True)
+    if form == "packed":
+        out = flash_attn_varlen_func(q.to(DEV), k.to(DEV), v.to(DEV), max_seqlen_q=max(lens), max_seqlen_k=max(lens),
+                                     cu_seqlens_k=cu_k.to(DEV), **kw)
+    else:
+        kc, vc, tables = paged_pool(gen, full, sum(-(-n // 64) for n in full) + 2, block_size=64)
+        slots = torch.cat([tables[b, torch.arange(n) // 64].long() * 64 + torch.arange(n) % 64 for b, n in enumerate(full)])
+        kc.view(-1, HK, D)[slots], vc.view(-1, HK, D)[slots] = k, v
+        bt = tables.to(DEV)
+        out = flash_attn_varlen_func(q[new].to(DEV), kc.to(DEV), vc.to(DEV), max_seqlen_q=max(lens), max_seqlen_k=max(full),
+                                     cu_seqlens_k=cu_k.to(DEV), block_table=bt, **kw)
+        if form != "paged":
+            kc2, vc2 = kc.clone(), vc.clone()
+            kc2.view(-1, HK, D)[slots[new]], vc2.view(-1, HK, D)[slots[new]] = 0, 0
+            kc2, vc2 = kc2.to(DEV), vc2.to(DEV)
+            fused = prefill_attention_store(q[new].to(DEV), k[new].to(DEV), v[new].to(DEV), kc2, vc2,
+                                            slots[new].to(torch.int32).to(DEV), max_seqlen_q=max(lens),
+                                            cu_seqlens_k=cu_k.to(DEV), block_table=bt, **kw)
+            assert torch.equal(fused, out) and torch.equal(kc2.cpu(), kc) and torch.equal(vc2.cpu(), vc)
+    attn_close(out, want, f"{form}, {rise}")

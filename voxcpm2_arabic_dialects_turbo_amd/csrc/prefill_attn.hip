@@ -1080,7 +1080,7 @@ __global__ __launch_bounds__(64 * RG * KS, 2) void prefill32_kernel(PrefillArgs 
   __shared__ __attribute__((aligned(1024))) uint8_t kt1[kTB];
   __shared__ __attribute__((aligned(1024))) uint8_t vt0[kTB];
   __shared__ __attribute__((aligned(1024))) uint8_t vt1[kTB];
-  __shared__ float red[KS == 2 ? 128 : 1];
+  __shared__ float red[KS == 2 ? 256 : 1];
   const pf32::Bufs bufs{kt0, kt1, vt0, vt1, red};
   int qt, b, g;
   grid_item(p, qt, b, g);

@@ -3,8 +3,8 @@
 //
 // An item is 32 RG query rows = (32 RG / G tokens) x (the G query heads of one kv head), as RG x KS waves: wave (rg, ks)
 // owns rows [32 rg, 32 rg + 32) and keys [64 / KS * ks, ...) of every 64-key tile. With KS = 1 a wave sees every key;
-// with KS = 2 two waves share a row block, each walking its half of every tile with an online softmax of its own, and
-// merge (O, m, l) through LDS at the end: half the instructions, LDS reads and MFMAs per wave and key tile, which is
+// with KS = 2 two waves share a row block, each walking its half of every tile from one row max (the first tile's, over
+// both halves), and merge (O, m, l) through LDS at the end: half the instructions, LDS reads and MFMAs per wave and key tile, which is
 // what a short grid's time is made of (a chain of key tiles walked by one wave per SIMD, bound by instruction issue).
 //
 // Per tile and wave: S^T[keys x 32 rows] = K Q^T (Q^T in registers; lane = (row col = lane & 31, half h = lane >> 5)),
@@ -52,7 +52,7 @@ struct Bufs {
   uint8_t* k1;
   uint8_t* v0;
   uint8_t* v1;
-  float* red;  // [4 waves][32] (two key halves)
+  float* red;  // [2][4 waves][32] (two key halves)
 };
 
 template <int SRC, int RG, int KS>
@@ -283,22 +283,23 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
       for (int i = 0; i < 16; ++i) t = fmaxf(t, sc[kt][i]);
     return xhalf_max(t) * c;
   };
-  auto pv = [&](const uint8_t* vd, const u32x4 (&pb)[2 * KT]) {
+  // The row max is that of the first tile, and p stays <= 2^62: ahead of a tile with a score more than 62 (log2 units) past
+  // it, or with a row's first key behind tiles without any, the row max moves (raise, a wave at a time). The scores are
+  // looked at beside the last four P V MFMAs of the tile before, which have no softmax left to hide, and compared behind
+  // its barrier. (Finding such a score by the row sum of its tile instead, with the accumulators already spoilt, and
+  // walking the item a second time: 1 x 1000 tokens 30.9 us with one such key, 15.1 this way, 14.5 both with none;
+  // 3 x 4096 314, 210 and 208, 210.)
+  float lim = 0.f;  // the score (not scaled) from which on the row max moves
+  auto raise = [&](const f32x16 (&sc)[KT]) {
+    const float tm = row_max(sc);
+    const bool up = tm > m + 8.f;
+    const float alpha = up ? fast_exp2(m - tm) : 1.f;  // exp2(-inf) = 0 on a row's first update
+    m = up ? tm : m;
+    lim = (m + 62.f) / c;
+    l *= alpha;
 #pragma unroll
-    for (int s = 0; s < 2 * KT; ++s)
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        const uint8_t* vp = vd + s * 4096 + (vrd ^ (uint32_t)(dt << 6));
-        const u32x2 lo = __builtin_bit_cast(u32x2, lds_read_tr16(reinterpret_cast<const uint16_t*>(vp)));
-        const u32x2 hi = __builtin_bit_cast(u32x2, lds_read_tr16(reinterpret_cast<const uint16_t*>(vp + 2048)));
-        acc[dt] = mfma_32x32x16(u32x4{lo[0], lo[1], hi[0], hi[1]}, pb[s], acc[dt]);
-      }
+    for (int dt = 0; dt < 4; ++dt) acc[dt] *= alpha;
   };
-  // The row max is that of the first tile: p stays <= 2^62 unless a later score passes it by 62 (log2 units), which a
-  // tile's partial row sum (at least its largest term) shows. Such an item, a rare one, is walked again below with a
-  // max per tile. (A branch for it inside the loop, moving the max and rescaling the accumulators, made the compiler
-  // keep two copies of them and move them across twice a tile.)
-  bool over = false;
   // KS = 2: the first tile's row max over both of its halves, so that p and its rounding are those of an unsplit row (and
   // the int8 output's two forms quantize the same values). The barrier waits for LDS only, not for tiles in flight.
   [[maybe_unused]] auto shared_max = [&](float x) -> float {
@@ -315,7 +316,6 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
   // rows for 32 bytes each), into buffers the first tiles leave free
   const int n = (kv_end + kBK - 1) / kBK;  // key tiles
   Place pl{bid, 0};                        // of the last K tile loaded
-  const Place pl0 = pl;
   bool ok = tile_ok(0, pl);                // whether the tile whose scores are held takes weight
   // The loop takes two tiles a round (fixed buffers: the compiler tells a tile's reads from the tiles in flight by the
   // arrays), with one tile before it where that leaves one: tile 0 then starts in the second buffers.
@@ -380,6 +380,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
     mask(sa, 0, ok);
     m = row_max(sa);
     if constexpr (KS == 2) m = shared_max(m);
+    lim = (m + 62.f) / c;
     if (RG != 2 || KS != 2) tile_barrier();
   }
   // One tile: the softmax of its scores (sc) beside the score MFMAs of the next tile (into sn) and its own first P V
@@ -395,7 +396,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
     constexpr int NE = 16 * KT;                     // elements per lane
     const float mu = m == -INFINITY ? 0.f : m;
     u32x4 pb[2 * KT];
-    float e[4], sum = 0.f;
+    float e[4], sum = 0.f, top = -INFINITY;
     auto element = [&](int x) {  // element x (key block x / 16, register x % 16) of the tile's probabilities
       e[x & 3] = fast_exp2(fmaf(sc[x >> 4][x & 15], c, -mu));
       if (x & 1) pb[x >> 3][(x >> 1) & 3] = pack_bf16x2(e[(x & 3) - 1], e[x & 3]);
@@ -442,12 +443,21 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
         read_v(i + AH - NS);
 #pragma unroll
       for (int x = i * NE / SPAN; x < (i + 1) * NE / SPAN && x < NE; ++x) element(x);
+      if (i >= NS + NP2 - 4) {  // this lane's largest score of the next tile (masked ones too)
+        constexpr int N4 = NE / 4;
+#pragma unroll
+        for (int x = 0; x < N4; ++x) {
+          const int y = (i - (NS + NP2 - 4)) * N4 + x;
+          top = fmaxf(top, sn[y >> 4][y & 15]);
+        }
+        asm volatile("" : "+v"(top));  // (here)
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
     l += sum;
-    over = over || !(sum <= 0x1p62f);  // also catches inf
     mask(sn, (t + 1) * kBK, ok);
     tile_barrier();
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(top > lim) != 0, 0)) raise(sn);
   };
   if (n > 0) {
     int t = 0;
@@ -471,46 +481,13 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
     };
 #pragma unroll
     for (int i = 0; i < 8; ++i) read_v(i);
-    const float sum = probs(sa, pb);
-    l += sum;
-    over = over || !(sum <= 0x1p62f);
+    l += probs(sa, pb);
 #pragma unroll
     for (int i = 0; i < 8 * KT; ++i) {
       acc[i & 3] = mfma_32x32x16(vf[i & 7], pb[i >> 2], acc[i & 3]);
       if (i + 8 < 8 * KT) read_v(i + 8);
     }
   }
-  if (n > 1 && __builtin_expect(__syncthreads_or(over), 0)) {  // (a first tile's p are at most 1)
-    // the item again, one tile at a time, the running max moving with every tile that passes it by more than 8
-    m = -INFINITY;
-    l = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
-    col_t = 0;
-    pl = pl0;
-    for (int t = 0; t < n; ++t) {
-      if (t > 0) pl = next_place(pl);
-      load_k(bufs.k0, t * kBK, pl);
-      load_v(bufs.v0, t * kBK, pl);
-      tile_barrier();
-      scores(bufs.k0, sa);
-      mask(sa, t * kBK, tile_ok(t * kBK, pl));
-      float tm = row_max(sa);
-      if constexpr (KS == 2) tm = shared_max(tm);
-      const bool up = tm > m + 8.f;
-      const float alpha = up ? fast_exp2(m - tm) : 1.f;  // exp2(-inf) = 0 on a row's first update
-      m = up ? tm : m;
-      u32x4 pb[2 * KT];
-      l = l * alpha + probs(sa, pb);
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) acc[dt] *= alpha;
-      pv(bufs.v0, pb);
-      __syncthreads();
-    }
-  }
-
   // ---- epilogue: normalize, bf16
   const float L = xhalf_sum(l);
   // the 32-dim blocks [d0, d0 + nd) of O, normalized by inv
@@ -548,7 +525,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
     uint8_t* const mine = w < 2 ? bufs.k0 + w * 8192 : bufs.k1 + (w - 2) * 8192;
     const int pw = w ^ RG;  // the partner
     const uint8_t* const theirs = pw < 2 ? bufs.k0 + pw * 8192 : bufs.k1 + (pw - 2) * 8192;
-    // (their p were taken against the same row max: the parts add up)
+    // (their p were taken against the same row max, and the parts add up, unless one of the waves has raised its own)
     __syncthreads();  // the last tile's reads are done
     auto merge = [&](auto half) {
       constexpr int OWN = 2 * decltype(half)::value, GIVE = 2 - OWN;
@@ -557,12 +534,30 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
         *reinterpret_cast<f32x4*>(mine + j * 1024 + lane * 16) =
             f32x4{acc[GIVE + (j >> 2)][(j & 3) * 4], acc[GIVE + (j >> 2)][(j & 3) * 4 + 1],
                   acc[GIVE + (j >> 2)][(j & 3) * 4 + 2], acc[GIVE + (j >> 2)][(j & 3) * 4 + 3]};
-      if (h == 0) bufs.red[w * 32 + col] = L;
+      if (h == 0) {
+        bufs.red[w * 32 + col] = L;
+        bufs.red[128 + w * 32 + col] = m;
+      }
       __syncthreads();
-      const float Ls = L + bufs.red[pw * 32 + col];
+      float Lt = bufs.red[pw * 32 + col];
+      const float mt = bufs.red[128 + pw * 32 + col];
       f32x4 y[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) y[j] = *reinterpret_cast<const f32x4*>(theirs + j * 1024 + lane * 16);
+      float Ls = L;
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(m != mt) != 0, 0)) {
+        const float M = fmaxf(m, mt);
+        const float a = m == M ? 1.f : fast_exp2(m - M), at = mt == M ? 1.f : fast_exp2(mt - M);
+        Ls *= a;
+        Lt *= at;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          y[j] *= at;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[OWN + (j >> 2)][(j & 3) * 4 + i] *= a;
+        }
+      }
+      Ls += Lt;
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll

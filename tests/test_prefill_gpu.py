@@ -945,3 +945,23 @@ def test_scores_rising_past_the_first_tile(form, lens, rise):
                                             cu_seqlens_k=cu_k.to(DEV), block_table=bt, **kw)
             assert torch.equal(fused, out) and torch.equal(kc2.cpu(), kc) and torch.equal(vc2.cpu(), vc)
     attn_close(out, want, f"{form}, {rise}")
+
+
+@pytest.mark.parametrize("lens,bs", [([20], 64), ([20, 7], 32), ([260, 33], 64), ([300, 129] + [40] * 12, 64),
+                                     ([64, 100, 250, 300, 410, 512, 80, 33], 64), ([300, 129] + [40] * 12, 32)],
+                         ids=["16-row waves", "per piece", "key halves", "128-row items", "rank order", "128 rows per piece"])
+def test_first_keys_behind_unmapped_blocks_score_far_below_zero(lens, bs):
+    """A context whose first 64 keys are unmapped and whose other scores all lie below -126 log2 units: a row max left at
+    zero would make every probability underflow. The oracle over the keys that are mapped."""
+    gen = torch.Generator().manual_seed(300 + len(lens))
+    nk = [n + 100 for n in lens]
+    kc, vc, tables = paged_pool(gen, nk, sum(-(-n // bs) for n in nk) + 2, block_size=bs)
+    u = torch.randn(HK, D, generator=gen)
+    q = (u.repeat_interleave(H // HK, dim=0) + 0.05 * torch.randn(sum(lens), H, D, generator=gen)).to(torch.bfloat16)
+    kc = (0.3 * kc.float() - 14 * u).to(torch.bfloat16)
+    t_gpu = tables.clone()
+    t_gpu[:, :64 // bs] = -1
+    out = flash_attn_varlen_func(q.to(DEV), kc.to(DEV), vc.to(DEV), _cu(lens).to(DEV), _cu(nk).to(DEV), max(lens), max(nk),
+                                 softmax_scale=SCALE, causal=True, block_table=t_gpu.to(DEV))
+    want = ref.varlen(q.float(), _cu(lens), _cu([n - 64 for n in nk]), k_cache=kc, v_cache=vc, block_tables=tables[:, 64 // bs:])
+    attn_close(out, want, "scores below zero")

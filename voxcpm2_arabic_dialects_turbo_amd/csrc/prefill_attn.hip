@@ -343,7 +343,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, int qt, int b
     bool big = false;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      const float mu = m[rt] == -INFINITY ? 0.f : m[rt];
+      // (a row without a key so far: its first ones fail the check, whatever their scores)
+      const float mu = m[rt] == -INFINITY ? -0x1p120f : m[rt];
       float s2[8];  // pair sums, added as a tree (depth 4, not a chain of 16 dependent adds)
       uint32_t pk[8];
 #pragma unroll

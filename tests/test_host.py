@@ -94,6 +94,77 @@ def test_step_staging_round_trips_dtypes_shapes_and_alignment():
     assert tb.tolist() == b.tolist()
 
 
+def test_step_staging_waits_for_the_copy_on_its_own_device(monkeypatch):
+    """A staging for device 1 while device 0 is current: the event that guards the buffer's next filling is recorded on
+    device 1's stream, where the copy runs, and whether a graph is being captured is asked of device 1. (Stand-ins for the
+    two devices; the copy's bytes are taken when its stream gets to it, that is when something waits for it.)"""
+    one, current, queued, asked = torch.device("cuda:1"), [0], {0: [], 1: []}, []
+
+    class Event:
+        device = None
+
+        def record(self, stream=None):
+            self.device = torch.device("cuda", current[0] if stream is None else stream)
+            self.behind = len(queued[self.device.index])
+
+        def synchronize(self):
+            for copy in queued[self.device.index][:self.behind]:
+                copy()
+
+    class Host:
+        def __init__(self, raw):
+            self.raw = raw
+
+        def numel(self):
+            return self.raw.size
+
+        def __getitem__(self, at):
+            return Host(self.raw[at])
+
+        def to(self, dev, non_blocking):
+            dst = Device(torch.empty(self.raw.size, dtype=torch.uint8))
+            queued[dev.index].append(lambda: dst.data.copy_(torch.from_numpy(self.raw)) if dst.left else None)
+            queued[dev.index].append(lambda: setattr(dst, "left", False))
+            return dst
+
+    class Device:
+        device, left = one, True
+
+        def __init__(self, data):
+            self.data = data
+
+        def view(self, dtype):
+            return self.data.view(dtype)
+
+    class use:
+        def __init__(self, dev):
+            self.index = dev.index
+
+        def __enter__(self):
+            self.prev, current[0] = current[0], self.index
+
+        def __exit__(self, *exc):
+            current[0] = self.prev
+
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "device", use)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: current[0] if device is None else device.index)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: asked.append(current[0]))
+    stage = runner.StepStaging("cuda:1")
+    for slot in stage._slots:
+        slot.raw = np.zeros(1024, dtype=np.uint8)
+        slot.host = Host(slot.raw)
+    got = []
+    for step in range(4):
+        view, = stage.layout([(np.int32, (5,))])
+        view[:] = step
+        got += stage.upload()
+    for copy in queued[1]:
+        copy()
+    assert [t.tolist() for t in got] == [[step] * 5 for step in range(4)]
+    assert asked == [1] * 4 and not queued[0]
+
+
 @pytest.mark.parametrize("first,count", [([3, 10, 0, 7], [2, 0, 3, 1]), ([5], [0]), ([], []), ([0, 0], [4, 4])])
 def test_runs_are_concatenated_aranges(first, count):
     f, c = np.array(first, dtype=np.int64), np.array(count, dtype=np.int64)

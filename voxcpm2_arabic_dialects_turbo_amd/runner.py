@@ -59,6 +59,14 @@ class RunnerTask:
 _ALIGN = 256  # every array starts at a multiple of 256 bytes, as separate device allocations would
 
 
+def _capturing(dev: torch.device) -> bool:
+    """Whether a HIP graph is being captured on ``dev``'s current stream."""
+    if dev.index is None:
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(dev):
+        return torch.cuda.is_current_stream_capturing()
+
+
 @dataclass
 class _Slot:
     host: torch.Tensor | None = None   # page-locked uint8 buffer
@@ -96,7 +104,7 @@ class StepStaging:
             parts.append((end, dtype, shape, n))
             end += -(-(dtype.itemsize * n) // _ALIGN) * _ALIGN
         need = max(end, _ALIGN)
-        persistent = dev.type == "cuda" and not torch.cuda.is_current_stream_capturing()
+        persistent = dev.type == "cuda" and not _capturing(dev)
         if persistent:
             slot = self._slots[self._turn]
             self._turn ^= 1
@@ -123,7 +131,8 @@ class StepStaging:
                 # (an event belongs to the device it was first recorded on: device "cuda" follows the current one)
                 if self._slot.done is None or self._slot.done.device != dst.device:
                     self._slot.done = torch.cuda.Event()
-                self._slot.done.record()
+                # behind the copy: on its device's stream, whichever device is current
+                self._slot.done.record(torch.cuda.current_stream(dst.device))
                 self._slot.pending = True
         else:
             dst = src.clone()

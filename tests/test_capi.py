@@ -6,6 +6,8 @@ from __future__ import annotations
 import ctypes
 import os
 import re
+import sys
+import types
 
 import pytest
 
@@ -355,3 +357,47 @@ def test_calls_module_takes_what_ctypes_takes():
         assert lib.vox_prefill_int8_workspace_bytes(*args) == size(*args)
     with pytest.raises(TypeError):
         lib.vox_store_kvcache(None)
+
+
+@pytest.mark.parametrize("version", [None, _lib.ABI_VERSION - 1, _lib.ABI_VERSION + 1])
+def test_calls_module_of_another_version_is_refused(monkeypatch, version):
+    """A CPython module compiled against another header would pass its arguments: it has to be rebuilt."""
+    old = types.ModuleType("_calls")
+    old.vox_store_kvcache, old.bind = (lambda *a: 0), (lambda addresses: None)
+    if version is not None:
+        old.ABI_VERSION = version
+    monkeypatch.setitem(sys.modules, _lib.__package__ + "._calls", old)
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(_lib.VoxAttnError, match="rebuild"):
+        _lib.load()
+
+
+@pytest.mark.parametrize("case", ["all", "module fails", "link fails"])
+def test_build_replaces_everything_or_nothing(monkeypatch, tmp_path, case):
+    """A failed step leaves the earlier library and module together. (Stand-ins for the compilers.)"""
+    from voxcpm2_arabic_dialects_turbo_amd import build
+
+    calls = str(tmp_path / os.path.basename(build.CALLS_PATH))
+    for name, path in (("PKG_DIR", tmp_path), ("BUILD_DIR", tmp_path / "o"), ("LIB_PATH", tmp_path / "lib.so"),
+                       ("PROBE_PATH", tmp_path / "probe.so"), ("CALLS_PATH", calls)):
+        monkeypatch.setattr(build, name, str(path))
+    outputs = [build.LIB_PATH, build.PROBE_PATH, calls, str(tmp_path / "_calls.so")]
+    for path in outputs:
+        with open(path, "w") as f:
+            f.write("old")
+
+    def run(cmd):
+        if (case == "module fails" and cmd[-1] == calls + ".tmp") or (case == "link fails" and build.PROBE_PATH in cmd[-1]):
+            raise RuntimeError("command failed")
+        with open(cmd[-1], "w") as f:
+            f.write("new")
+
+    monkeypatch.setattr(build, "_run", run)
+    monkeypatch.setattr(build, "hipcc", lambda: "hipcc")
+    if case.endswith("fails"):
+        with pytest.raises(RuntimeError):
+            build.build()
+    else:
+        build.build()
+    found = [open(p).read() if os.path.exists(p) else None for p in outputs]
+    assert found == (["new", "new", "new", None] if case == "all" else ["old"] * 4)

@@ -9,6 +9,7 @@ hands out are valid in the library.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 import threading
 
@@ -92,6 +93,19 @@ _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 
 
+def _calls_module():
+    """The CPython module. It holds the signatures of the header it was compiled with, so it has to be of the library's
+    version."""
+    try:
+        calls = importlib.import_module("._calls", __package__)
+    except ImportError as e:
+        raise VoxAttnError(f"{e}: run `python -m voxcpm2_arabic_dialects_turbo_amd.build`") from e
+    version = getattr(calls, "ABI_VERSION", None)
+    if version != ABI_VERSION:
+        raise VoxAttnError(f"_calls module ABI {version} != {ABI_VERSION}: rebuild the library")
+    return calls
+
+
 def load() -> ctypes.CDLL:
     """Opens libvoxattn.so once per process and declares every entry point's signature."""
     global _lib
@@ -113,14 +127,11 @@ def load() -> ctypes.CDLL:
                 raise VoxAttnError(f"libvoxattn ABI {lib.vox_abi_version()} != {ABI_VERSION}: rebuild the library")
             # the entry points called on every layer, through the CPython module: the same functions, without ctypes'
             # argument conversion
-            try:
-                from . import _calls
-            except ImportError as e:
-                raise VoxAttnError(f"_calls.so ({e}): run `python -m voxcpm2_arabic_dialects_turbo_amd.build`") from e
-            fast = [n for n in EXPORTS if hasattr(_calls, n)]
-            _calls.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in fast})
+            calls = _calls_module()
+            fast = [n for n in EXPORTS if hasattr(calls, n)]
+            calls.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in fast})
             for n in fast:
-                setattr(lib, n, getattr(_calls, n))
+                setattr(lib, n, getattr(calls, n))
             _lib = lib
     return _lib
 

@@ -1,7 +1,7 @@
 """Builds libvoxattn.so in-tree with hipcc for gfx950 (run as ``python -m voxcpm2_arabic_dialects_turbo_amd.build``).
 
 The attention library is one shared library, C ABI only (include/vox_attn.h): no torch headers, no pybind. The
-sources compile in parallel and link into ``voxcpm2_arabic_dialects_turbo_amd/libvoxattn.so``. Beside it, ``_calls.so`` is
+sources compile in parallel and link into ``voxcpm2_arabic_dialects_turbo_amd/libvoxattn.so``. Beside it, ``_calls`` is
 the CPython module through which the operators call it (csrc/host_calls.cpp, host code only), and
 ``libvoxprobe.so`` (include/vox_probe.h) holds the memory-rate probes bench.py runs; the attention path never loads
 it. Packed FP32 VALU instructions are disabled for
@@ -26,8 +26,8 @@ LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 SOURCES = ["store_kvcache.hip", "decode_attn.hip", "prefill_attn.hip", "quantize_rows.hip", "kv_copy.hip", "capi.hip"]
 PROBE_PATH = os.path.join(PKG_DIR, "libvoxprobe.so")
 PROBE_SOURCES = ["bench_probe.hip"]
-# the CPython entry to the C ABI (host code only)
-CALLS_PATH = os.path.join(PKG_DIR, "_calls.so")
+# the CPython entry to the C ABI (host code only), for the interpreter that builds it
+CALLS_PATH = os.path.join(PKG_DIR, "_calls" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 CALLS_SOURCE = "host_calls.cpp"
 ARCH = "gfx950"
 
@@ -64,14 +64,18 @@ def _run(cmd: list[str]) -> None:
 
 
 def build(verbose: bool = False) -> str:
-    """Compiles every source and links libvoxattn.so and libvoxprobe.so; returns the attention library's path.
-    Always rebuilds."""
+    """Compiles every source and links libvoxattn.so and libvoxprobe.so and the CPython module; returns the attention
+    library's path. Always rebuilds; what was built before is replaced only when everything compiles, all of it."""
     cc = hipcc()
     os.makedirs(BUILD_DIR, exist_ok=True)
     cmds = []
     for src in SOURCES + PROBE_SOURCES:
         obj = os.path.join(BUILD_DIR, src.replace(".hip", ".o"))
         cmds.append([cc, *compile_flags(), "-c", os.path.join(CSRC, src), "-o", obj])
+    cxx = os.environ.get("CXX") or shutil.which("g++") or cc
+    cmds.append([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
+                 f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, CALLS_SOURCE), "-o", CALLS_PATH + ".tmp"])
+    built = [LIB_PATH, PROBE_PATH, CALLS_PATH]
     with ThreadPoolExecutor(max_workers=min(len(cmds), os.cpu_count() or 1)) as ex:
         for cmd, fut in zip(cmds, [ex.submit(_run, c) for c in cmds]):
             if verbose:
@@ -79,13 +83,12 @@ def build(verbose: bool = False) -> str:
             fut.result()
     for path, srcs in ((LIB_PATH, SOURCES), (PROBE_PATH, PROBE_SOURCES)):
         objs = [os.path.join(BUILD_DIR, src.replace(".hip", ".o")) for src in srcs]
-        tmp = path + ".tmp"
-        _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])
-        os.replace(tmp, path)
-    cxx = os.environ.get("CXX") or shutil.which("g++") or cc
-    _run([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
-          f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, CALLS_SOURCE), "-o", CALLS_PATH + ".tmp"])
-    os.replace(CALLS_PATH + ".tmp", CALLS_PATH)
+        _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", path + ".tmp"])
+    for old in (CALLS_PATH, os.path.join(PKG_DIR, "_calls.so")):  # (a module of another build is not left beside these)
+        if old not in built and os.path.exists(old):
+            os.remove(old)
+    for path in built:
+        os.replace(path + ".tmp", path)
     return LIB_PATH
 
 

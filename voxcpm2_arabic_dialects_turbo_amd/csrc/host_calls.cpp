@@ -106,4 +106,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods, nul
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__calls(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__calls(void) {
+  PyObject* m = PyModule_Create(&module);
+  // the header's version: the signatures above are those of a library of the same one
+  if (m && PyModule_AddIntConstant(m, "ABI_VERSION", VOX_ABI_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -372,9 +372,18 @@ def test_calls_module_of_another_version_is_refused(monkeypatch, version):
         _lib.load()
 
 
-@pytest.mark.parametrize("case", ["all", "module fails", "link fails"])
+def test_without_the_calls_module_the_entry_points_are_the_ctypes_ones(monkeypatch):
+    monkeypatch.setitem(sys.modules, _lib.__package__ + "._calls", None)  # (as if there were none)
+    monkeypatch.setattr(_lib, "_lib", None)
+    lib = _lib.load()
+    assert isinstance(lib.vox_prefill_attn, ctypes._CFuncPtr) and lib.vox_prefill_attn.argtypes
+    assert lib.vox_store_kvcache(None, 16, 256, 256, 16, 16, 10, 16, 4, 2, 128, None) == _lib.VOX_EINVAL
+
+
+@pytest.mark.parametrize("case", ["all", "no headers", "module fails", "link fails"])
 def test_build_replaces_everything_or_nothing(monkeypatch, tmp_path, case):
-    """A failed step leaves the earlier library and module together. (Stand-ins for the compilers.)"""
+    """A failed step leaves the earlier library and module together; a build without Python's headers leaves no module of
+    an earlier one beside the new library. (Stand-ins for the compilers.)"""
     from voxcpm2_arabic_dialects_turbo_amd import build
 
     calls = str(tmp_path / os.path.basename(build.CALLS_PATH))
@@ -394,10 +403,11 @@ def test_build_replaces_everything_or_nothing(monkeypatch, tmp_path, case):
 
     monkeypatch.setattr(build, "_run", run)
     monkeypatch.setattr(build, "hipcc", lambda: "hipcc")
+    monkeypatch.setattr(build, "_python_include", lambda: None if case == "no headers" else "/include")
     if case.endswith("fails"):
         with pytest.raises(RuntimeError):
             build.build()
     else:
         build.build()
     found = [open(p).read() if os.path.exists(p) else None for p in outputs]
-    assert found == (["new", "new", "new", None] if case == "all" else ["old"] * 4)
+    assert found == {"all": ["new", "new", "new", None], "no headers": ["new", "new", None, None]}.get(case, ["old"] * 4)

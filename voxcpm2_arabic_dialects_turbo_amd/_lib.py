@@ -94,10 +94,12 @@ _lib: ctypes.CDLL | None = None
 
 
 def _calls_module():
-    """The CPython module. It holds the signatures of the header it was compiled with, so it has to be of the library's
-    version."""
+    """The CPython module of this interpreter (None: the build had no Python headers, or was another interpreter's). It
+    holds the signatures of the header it was compiled with, so it has to be of the library's version."""
     try:
         calls = importlib.import_module("._calls", __package__)
+    except ModuleNotFoundError:
+        return None
     except ImportError as e:
         raise VoxAttnError(f"{e}: run `python -m voxcpm2_arabic_dialects_turbo_amd.build`") from e
     version = getattr(calls, "ABI_VERSION", None)
@@ -125,13 +127,14 @@ def load() -> ctypes.CDLL:
                 fn.argtypes = args
             if lib.vox_abi_version() != ABI_VERSION:
                 raise VoxAttnError(f"libvoxattn ABI {lib.vox_abi_version()} != {ABI_VERSION}: rebuild the library")
-            # the entry points called on every layer, through the CPython module: the same functions, without ctypes'
-            # argument conversion
+            # the entry points called on every layer, through the CPython module where it is built: the same functions,
+            # without ctypes' argument conversion
             calls = _calls_module()
-            fast = [n for n in EXPORTS if hasattr(calls, n)]
-            calls.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in fast})
-            for n in fast:
-                setattr(lib, n, getattr(calls, n))
+            if calls is not None:
+                fast = [n for n in EXPORTS if hasattr(calls, n)]
+                calls.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in fast})
+                for n in fast:
+                    setattr(lib, n, getattr(calls, n))
             _lib = lib
     return _lib
 

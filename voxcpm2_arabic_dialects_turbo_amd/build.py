@@ -2,7 +2,8 @@
 
 The attention library is one shared library, C ABI only (include/vox_attn.h): no torch headers, no pybind. The
 sources compile in parallel and link into ``voxcpm2_arabic_dialects_turbo_amd/libvoxattn.so``. Beside it, ``_calls`` is
-the CPython module through which the operators call it (csrc/host_calls.cpp, host code only), and
+the CPython module through which the operators call it (csrc/host_calls.cpp, host code only; without Python's headers it
+is left out and the same entry points are called through ctypes), and
 ``libvoxprobe.so`` (include/vox_probe.h) holds the memory-rate probes bench.py runs; the attention path never loads
 it. Packed FP32 VALU instructions are disabled for
 device code (``-packed-fp32-ops``); hipcc's host pass warns that it does not know that feature, which is harmless.
@@ -63,6 +64,12 @@ def _run(cmd: list[str]) -> None:
         print(text, file=sys.stderr)
 
 
+def _python_include() -> str | None:
+    """The directory of Python.h, None where Python's headers are not installed."""
+    path = sysconfig.get_paths()["include"]
+    return path if os.path.exists(os.path.join(path, "Python.h")) else None
+
+
 def build(verbose: bool = False) -> str:
     """Compiles every source and links libvoxattn.so and libvoxprobe.so and the CPython module; returns the attention
     library's path. Always rebuilds; what was built before is replaced only when everything compiles, all of it."""
@@ -72,10 +79,15 @@ def build(verbose: bool = False) -> str:
     for src in SOURCES + PROBE_SOURCES:
         obj = os.path.join(BUILD_DIR, src.replace(".hip", ".o"))
         cmds.append([cc, *compile_flags(), "-c", os.path.join(CSRC, src), "-o", obj])
-    cxx = os.environ.get("CXX") or shutil.which("g++") or cc
-    cmds.append([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
-                 f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, CALLS_SOURCE), "-o", CALLS_PATH + ".tmp"])
-    built = [LIB_PATH, PROBE_PATH, CALLS_PATH]
+    include = _python_include()
+    built = [LIB_PATH, PROBE_PATH]
+    if include is not None:
+        cxx = os.environ.get("CXX") or shutil.which("g++") or cc
+        cmds.append([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", f"-I{include}",
+                     os.path.join(CSRC, CALLS_SOURCE), "-o", CALLS_PATH + ".tmp"])
+        built.append(CALLS_PATH)
+    else:
+        print("Python.h not found: the operators will call the library through ctypes", file=sys.stderr)
     with ThreadPoolExecutor(max_workers=min(len(cmds), os.cpu_count() or 1)) as ex:
         for cmd, fut in zip(cmds, [ex.submit(_run, c) for c in cmds]):
             if verbose:

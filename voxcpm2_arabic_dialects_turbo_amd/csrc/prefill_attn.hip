@@ -143,7 +143,9 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, int qt, int b
   if (KV != kPacked) nk = min(nk, p.max_blocks * p.block_size);  // keys the block table can address
   const int G = p.group;
   const int BQ = ROWS / G;  // query tokens per workgroup
-  if (qt * BQ >= nq || (p.skip_single && nq == 1)) return;  // (one-query rows: the decode kernel's, in varlen mode)
+  if (qt * BQ >= nq) return;
+  if constexpr (KV != kPacked)
+    if (p.skip_single && nq == 1) return;  // (one-query rows: the decode kernel's, in paged varlen mode)
   if constexpr (!QUANT && (KV == kPacked || KV == kPagedTilesRows))
     if (gz >= p.num_kv_heads) return;  // a workgroup that only copies (a riding store)
 

@@ -1274,7 +1274,7 @@ hipError_t launch_prefill(const PrefillArgs& a0, int max_seqlen_q, hipStream_t s
   // ... in a plain causal grid over paged tiles or packed keys by the workgroups of each sequence's first half of the q
   // tiles, the ones with the short chains (one prompt of 237 tokens: the copy behind the longest chain cost 0.7 us)
   auto store_by_light = [&](int64_t q_tiles) {
-    if (a.store_rows <= 0 || !a.causal || a.xcd_order || q_tiles < 8 || (a.block_tables && a.block_size % kBK)) return;
+    if (a.store_rows <= 0 || !a.causal || a.xcd_order || q_tiles < 8) return;
     a.store_light = (int)((q_tiles + 1) / 2);
     const int64_t wgs = a.store_light * (int64_t)a.batch * a.num_kv_heads;
     a.store_wgs = (int)(wgs < 256 ? wgs : 256);

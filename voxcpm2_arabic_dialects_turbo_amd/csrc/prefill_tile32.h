@@ -62,7 +62,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
   constexpr int KT = 2 / KS;         // 32-key blocks per wave and tile
   constexpr int WR = kBK / NW;       // tile rows a wave loads
   constexpr int NP = WR / 4;         // its load instructions (4 rows each) for K, and for V
-  static_assert(KS == 1 || (KS == 2 && NW == 4), "a wave takes 32-key blocks; the merge uses 8 KB a wave");
+  static_assert(NW == 4 && (KS == 1 || KS == 2), "a wave takes 32-key blocks; the merge uses 8 KB a wave");
 
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int rg = w % RG, ks = w / RG;
@@ -328,7 +328,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
   f32x16 sa[KT], sb[KT];
   uint16_t* op = p.out + ((int64_t)q0 + tq) * p.out_row_stride + head * kD + h * 8;  // this lane's output row
   if (n > 0) {
-    uint8_t* const qbuf = RG == 2 ? vsecond + rg * 8192 : (rg < 2 ? ksecond + rg * 8192 : vsecond + (rg - 2) * 8192);
+    uint8_t* const qbuf = KS == 2 ? vsecond + rg * 8192 : (rg < 2 ? ksecond + rg * 8192 : vsecond + (rg - 2) * 8192);
     constexpr int NQ = 8 / KS;  // pieces (4 rows) this wave loads of its row block
     // (rows past the sequence or the limit read as zeros; their output is not stored)
     const int64_t tok0 = (int64_t)q0 + (int64_t)qt * BQ;
@@ -363,7 +363,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
     }
     load_k(kfirst, 0, pl);
     load_v(vfirst, 0, pl);
-    if (RG == 2 && n > 1) {
+    if (KS == 2 && n > 1) {
       pl = next_place(pl);
       load_k(ksecond, kBK, pl);
     }
@@ -372,7 +372,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
     tile_barrier();
 #pragma unroll
     for (int s = 0; s < 8; ++s) qop[s] = *reinterpret_cast<const u32x4*>(qbuf + (frag ^ (uint32_t)(s << 5)));
-    if (RG != 2 && n > 1) {
+    if (KS == 1 && n > 1) {
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave has its query rows
       pl = next_place(pl);
       load_k(ksecond, kBK, pl);
@@ -383,7 +383,7 @@ __device__ __forceinline__ void tile(const PrefillArgs& p, const int qt, const i
     if constexpr (KS == 2) m = shared_max(m);
     if (n > 1) {  // (an item of one tile has no next one to wait for: 12 layers of 250 x 16 rows 150.7 -> 148.5 us)
       lim = (m + 62.f) * rc;
-      if (RG != 2 || KS != 2) tile_barrier();
+      if constexpr (KS == 1) tile_barrier();
     }
   }
   // One tile: the softmax of its scores (sc) beside the score MFMAs of the next tile (into sn) and its own first P V

@@ -147,7 +147,7 @@ def test_decode_sparse_batch_of_mostly_empty_rows(grid):
                          ids=["1x16384", "4x4096", "16x300+8192", "mixed"])
 def test_decode_few_long_sequences(lens):
     """Few sequences, some far longer than a workgroup's share of the steps: the launch then uses fewer workgroups
-    (no sequence is cut into more than about 32 partials) and the merge kernel folds the partials of one sequence in
+    (no sequence of up to 64 is cut into more than about 64 partials, of more than that 32) and the merge kernel folds the partials of one sequence in
     several batches of loads."""
     gen = torch.Generator().manual_seed(40)
     pool = sum((max(n, 1) + BLOCK - 1) // BLOCK for n in lens) + 4
@@ -164,7 +164,7 @@ def test_decode_few_long_sequences(lens):
                               "65 with empty rows"])
 def test_decode_merge_forms(lens):
     """The merge with four workgroups per sequence (up to 64 sequences) and with one (beyond), over one partial, as many
-    as a wave takes in a batch and more (6000 tokens in up to 62 ranges), and ranges of four 16-token steps and fewer."""
+    as a wave takes in a batch and more (6000 tokens in up to 62 ranges, in up to 30 beyond 64 sequences)."""
     gen = torch.Generator().manual_seed(90 + len(lens) + lens[0])
     kc, vc, tables = paged_pool(gen, [max(n, 1) for n in lens], sum(-(-max(n, 1) // BLOCK) for n in lens) + 2)
     (_, _), out = _check(randn(gen, len(lens), H, D), kc, vc, lens, tables, f"{len(lens)} sequences")

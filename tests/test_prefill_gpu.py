@@ -240,9 +240,9 @@ def test_prefill_closed_forms_identical_keys():
 
 
 def test_prefill_scores_growing_across_key_tiles():
-    """Later key tiles score far above the first (log2-scaled scores hundreds of units higher), which sends those
-    tiles down the recompute-with-their-max path of the softmax; the result still matches the oracle, with no
-    overflow, for packed and paged keys."""
+    """Later key tiles score far above the first (log2-scaled scores hundreds of units higher) in one prompt of 300 tokens
+    (38 items of 64 rows: two row blocks x two key halves), which raises the row max ahead of those tiles, in each half by
+    itself; the result still matches the oracle, with no overflow, for packed and paged keys."""
     gen = torch.Generator().manual_seed(58)
     L = 300
     u = torch.randn(HK, D, generator=gen)  # a direction per kv group; every query leans along its group's
@@ -273,9 +273,8 @@ def test_prefill_scores_growing_across_key_tiles():
 @pytest.mark.parametrize("paged", [False, True])
 def test_scores_growing_across_key_tiles_in_the_32_row_form(paged):
     """The same growing scores in a grid above 2048 workgroups (one 2100-token sequence beside seven short ones:
-    132 q tiles x 8 x 2), which takes the 4-wave x 32-row form and its pipelined loop, where a tile whose scores
-    pass the running max is redone at the start of the next step; about every second key tile of the long sequence
-    takes that path."""
+    132 q tiles x 8 x 2), which takes items of 128 rows, 4 waves of a 32-row block each; about every second key tile of
+    the long sequence raises the row max."""
     gen = torch.Generator().manual_seed(59)
     lens = [2100] + [int(x) for x in torch.randint(20, 120, (7,), generator=gen)]
     T = sum(lens)
@@ -909,18 +908,21 @@ _RISES = {"first tile": {5: 12.0}, "second tile": {64: 12.0}, "one key half": {7
 @pytest.mark.parametrize("rise", list(_RISES))
 @pytest.mark.parametrize("lens", [[150], [300], [333, 192, 257], [300, 129] + [40] * 12, [64, 100, 250, 300, 410, 512, 80, 33]],
                          ids=["16-row waves", "key halves", "3 of key halves", "128-row items", "rank order"])
-@pytest.mark.parametrize("form", ["packed", "paged", "riding", "prefix"])
+@pytest.mark.parametrize("form", ["packed", "paged", "riding", "prefix", "mixed"])
 def test_scores_rising_past_the_first_tile(form, lens, rise):
     """Keys whose scores pass the first tile's max by more than 62 log2 units, in each half of a tile, in the last tile,
     in every tile, far beyond 2^127, and falling ones, over every bf16 form: the tiles of 16-row waves (redone with their
     max) and of 32-row blocks (the row max raised ahead of the tile), from packed rows, cached keys, and new rows beside
-    cached ones (a riding store, with and without a prefix). Against the oracle; the cached forms bit for bit alike."""
+    cached ones (a riding store, with and without a prefix, and beside decode rows). Against the oracle; the cached forms
+    bit for bit alike."""
     from voxcpm2_arabic_dialects_turbo_amd.ops import prefill_attention_store
 
     gen = torch.Generator().manual_seed(200 + len(lens))
     prefix = 50 if form == "prefix" else 0
     high = {max(lens) + prefix - 1: 12.0} if rise == "last key" else _RISES[rise]
     full = [n + prefix for n in lens]
+    if form == "mixed":
+        lens, full = lens + [1] * 12, full + [200] * 12
     q, k, v = _with_high_keys(gen, full, high)
     new = torch.cat([torch.arange(at - n, at) for n, at in zip(lens, np.cumsum(full).tolist())])  # rows of the new tokens
     cu_q, cu_k = _cu(lens), _cu(full)
@@ -965,3 +967,33 @@ def test_first_keys_behind_unmapped_blocks_score_far_below_zero(lens, bs):
                                  softmax_scale=SCALE, causal=True, block_table=t_gpu.to(DEV))
     want = ref.varlen(q.float(), _cu(lens), _cu([n - 64 for n in nk]), k_cache=kc, v_cache=vc, block_tables=tables[:, 64 // bs:])
     attn_close(out, want, "scores below zero")
+
+
+@pytest.mark.parametrize("lens", [[300, 7], [300] + [40] * 13], ids=["key halves", "128-row items"])
+@pytest.mark.parametrize("rise", [None, 100, 4095, 4096, 4250])
+def test_32_row_blocks_over_tables_wider_than_64_columns(lens, rise):
+    """New tokens behind 4000 cached ones in 64-token blocks: 68 table columns, the ones past 63 read tile by tile. Plain
+    and with one key far above the others on either side of column 64; with the riding store bit for bit alike."""
+    from voxcpm2_arabic_dialects_turbo_amd.ops import prefill_attention_store
+
+    gen = torch.Generator().manual_seed(400 + len(lens))
+    nq, nk, kc, vc, tables, q, k, v, slots = _step_with_new_rows(gen, lens, [4000] + [70] * (len(lens) - 1), [], HK, 64)
+    assert tables.shape[1] == 68
+    u = torch.randn(HK, D, generator=gen)
+    q = (q.float() * 0.3 + u.repeat_interleave(H // HK, dim=0).to(DEV)).to(torch.bfloat16)
+    if rise is not None:
+        high = (u * 12).to(torch.bfloat16)
+        kc[tables[0, rise // 64], rise % 64] = high
+        if rise >= 4000:
+            k[rise - 4000] = high.to(DEV)
+    cu_q, cu_k, bt, sl = _cu(nq).to(DEV), _cu(nk).to(DEV), tables.to(DEV), slots.to(DEV)
+    kc1, vc1 = kc.to(DEV), vc.to(DEV)
+    kc2, vc2 = kc1.clone(), vc1.clone()
+    kw = dict(cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=max(nq), softmax_scale=SCALE, block_table=bt)
+    fused = prefill_attention_store(q, k, v, kc1, vc1, sl, **kw)
+    store_kvcache(k, v, kc2, vc2, sl)
+    two = flash_attn_varlen_func(q, kc2, vc2, max_seqlen_k=max(nk), causal=True, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(fused, two) and torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
+    attn_close(two, ref.varlen(q.float().cpu(), _cu(nq), _cu(nk), k_cache=kc2.cpu(), v_cache=vc2.cpu(), block_tables=tables),
+               "68 columns")

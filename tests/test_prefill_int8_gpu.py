@@ -462,3 +462,30 @@ def test_paged_int8_prefill_with_the_store_riding_in_it_equals_store_then_prefil
     torch.cuda.synchronize()
     assert torch.equal(codes, codes2) and torch.equal(scales, scales2), f"{case}: int8 output differs"
     assert torch.equal(kc1, kc2) and torch.equal(vc1, vc2), f"{case}: caches differ from store_kvcache's"
+
+
+@pytest.mark.parametrize("lens", [[20, 40], [150], [333, 150, 271, 500, 9, 310]], ids=["short", "16-row waves", "two-pass"])
+@pytest.mark.parametrize("fused", [True, False])
+def test_int8_scores_rising_past_the_first_tile(lens, fused, monkeypatch):
+    """Keys scoring hundreds of log2 units above the first tile's, one in each of two later tiles, through the fused int8
+    output (tiles redone with their max) and, where the shape has it, the two-pass one (the row max raised ahead)."""
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(90 + len(lens))
+    T = sum(lens)
+    two_pass = lib.vox_prefill_int8_workspace_bytes(T, len(lens), max(lens), H, HK, D, 1) > 0
+    assert two_pass == (len(lens) > 2)
+    if fused:
+        monkeypatch.setattr(lib, "vox_prefill_int8_workspace_bytes", lambda *a: 0)
+    u = torch.randn(HK, D, generator=gen)
+    q = (u.repeat_interleave(H // HK, dim=0) + 0.3 * torch.randn(T, H, D, generator=gen)).to(torch.bfloat16)
+    k, v = randn(gen, T, HK, D), randn(gen, T, HK, D)
+    at = 0
+    for n in lens:
+        for pos, f in ((70, 9.0), (130, 16.0)):
+            if pos < n:
+                k[at + pos] = (u * f).to(torch.bfloat16)
+        at += n
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    out = varlen_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu_seqlens_q=cu.to(DEV), cu_seqlens_k=cu.to(DEV),
+                           max_seqlen_q=max(lens), softmax_scale=SCALE, causal=True, quant=True)
+    _check(out, ref.varlen(q.float(), cu, cu, k=k, v=v), "rising scores")

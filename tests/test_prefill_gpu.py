@@ -997,3 +997,25 @@ def test_32_row_blocks_over_tables_wider_than_64_columns(lens, rise):
     assert torch.equal(fused, two) and torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
     attn_close(two, ref.varlen(q.float().cpu(), _cu(nq), _cu(nk), k_cache=kc2.cpu(), v_cache=vc2.cpu(), block_tables=tables),
                "68 columns")
+
+
+@pytest.mark.parametrize("lens", [[300, 150], [300] + [180] * 13], ids=["key halves", "128-row items"])
+def test_riding_store_over_a_table_narrower_than_the_keys(lens):
+    """No cached keys and more new ones than the table's two columns address: the keys past the table take no part, and
+    the queries are aligned with the last one that does, as over the stored caches (outputs bit for bit alike)."""
+    from voxcpm2_arabic_dialects_turbo_amd.ops import prefill_attention_store
+
+    gen = torch.Generator().manual_seed(500 + len(lens))
+    nq, nk, kc, vc, tables, q, k, v, slots = _step_with_new_rows(gen, lens, [0] * len(lens), [], HK, 64)
+    cu, bt, sl = _cu(nq).to(DEV), tables[:, :2].contiguous().to(DEV), slots.to(DEV)
+    kc1, vc1 = kc.to(DEV), vc.to(DEV)
+    kc2, vc2 = kc1.clone(), vc1.clone()
+    kw = dict(cu_seqlens_q=cu, cu_seqlens_k=cu, max_seqlen_q=max(nq), softmax_scale=SCALE, block_table=bt)
+    fused = prefill_attention_store(q, k, v, kc1, vc1, sl, **kw)
+    store_kvcache(k, v, kc2, vc2, sl)
+    two = flash_attn_varlen_func(q, kc2, vc2, max_seqlen_k=max(nk), causal=True, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(fused, two) and torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
+    want = ref.varlen(q[nq[0] - 128:nq[0]].float().cpu(), _cu([128]), _cu([128]), k=k[:128].cpu(), v=v[:128].cpu())
+    attn_close(two[nq[0] - 128:nq[0]], want, "the last 128 queries of the first sequence")
+    assert not two[:nq[0] - 128].any()

@@ -144,7 +144,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, int qt, int b
   const int G = p.group;
   const int BQ = ROWS / G;  // query tokens per workgroup
   if (qt * BQ >= nq) return;
-  if constexpr (KV != kPacked)
+  if constexpr (!QUANT && KV != kPacked && KV != kPagedTilesRows)
     if (p.skip_single && nq == 1) return;  // (one-query rows: the decode kernel's, in paged varlen mode)
   if constexpr (!QUANT && (KV == kPacked || KV == kPagedTilesRows))
     if (gz >= p.num_kv_heads) return;  // a workgroup that only copies (a riding store)

@@ -560,7 +560,8 @@ int vox_prefill_attn_store_paged(const void* q, int64_t q_row_stride, const void
   const bool fold_mixed = attend && num_tokens > 0 && max_seqlen_q > 1 && vec16 && decode_rows &&
                           vox::mixed_launch_fits(a, num_kv_heads);
   // without the decode rows' workspace the prefill kernel takes every row: the store rides in its launch as in the
-  // packed form (the last workgroups copy the rows), the new keys read from the rows
+  // packed form (workgroups that have done their item, or have none, copy the rows beside the others' reads), and the
+  // new keys are read from the rows alone
   const bool fold_plain = attend && num_tokens > 0 && vec16 && !decode_rows && block_size % 64 == 0;
   if (fold_plain) {
     a.k_src = (const uint16_t*)key;

@@ -7,9 +7,12 @@
 // j <= nk - nq + i (bottom-right aligned), o = softmax(scale * q k^T) v in fp32, stored as bf16. Keys come from the
 // paged cache through block_tables, or from packed [Tk, HK, D] rows when there is no block table.
 //
-// gfx950 mapping. A workgroup owns 128 query rows = (128 / G tokens) x (the G query heads of one kv head), as 4 waves
-// of 32 rows on grids above 2048 workgroups, else 8 waves of 16; grids that fit two workgroups per CU take 64-row
-// workgroups of 4 waves of 16. GQA shares every K/V tile across the group's heads.
+// gfx950 mapping. A workgroup owns 64 or 128 query rows = (rows / G tokens) x (the G query heads of one kv head); GQA
+// shares every K/V tile across the group's heads. bf16 items over packed keys or paged blocks of a multiple of 64
+// tokens: of 128 rows, and of 64 rows where the sequences are long enough for key halves, as 32-row blocks
+// (prefill32_kernel, prefill_tile32.h); 64-row items of shorter sequences (grids that fit two workgroups per CU), of the
+// rank-major and the mixed grids as 4 waves of 16 rows (prefill_kernel, this file). Other block sizes: 128-row items as 4
+// waves of 32 rows on grids above 2048 workgroups, else 8 waves of 16, and 64-row ones as above.
 // Per 64-key tile K and V go from global memory straight into LDS (range-checked buffer loads with the lds bit: no
 // register staging; rows past the keys and unmapped blocks read as zeros), double-buffered, with the 16-byte chunks
 // of each 256-byte row permuted so that the fragment reads meet no bank conflicts; each wave computes
@@ -77,9 +80,7 @@ enum KvSource { kPacked = 0, kPagedTiles = 1, kPagedPieces = 2, kPagedTilesNew =
 // a tile loop of their own that reads only the rows.
 constexpr bool kv_tiles(int kv) { return kv == kPagedTiles || kv == kPagedTilesNew || kv == kPagedTilesRows; }
 
-// NW waves per KV group, each owning RT 16-row blocks of the 128 query rows: 4 waves x 32 rows keep the LDS reads per
-// MFMA low (the largest grids); 8 waves x 16 rows halve each wave's work per key tile, which shortens a workgroup's
-// chain of key tiles (smaller grids, where the longest chains end the launch).
+// NW waves per KV group, each owning RT 16-row blocks of the item's query rows.
 // The double-buffered K and V tiles of the direct-to-LDS path ([NH] = one per KV-group half), four distinct __shared__
 // arrays of the kernel: the compiler can then tell a tile's reads from the next tile's in-flight DMA writes (a
 // mixed launch's decode workgroups use the same arrays for their own state).
@@ -1037,8 +1038,7 @@ __device__ __forceinline__ void grid_item(const PrefillArgs& p, int& qt, int& b,
 }
 
 // Waves per SIMD the registers must allow: two 4-wave workgroups per CU (their 64 KB of LDS each fits twice), two
-// 8-wave ones (at most 128 VGPRs: the riding store's paged form would take 132 and hold one workgroup per CU, which
-// ran the 44 x 46-token step's 264 workgroups in two rounds, 15.4 -> 17.6 us), one int8 workgroup (128 KB of LDS).
+// 8-wave ones (block sizes that are no multiple of 64; at most 128 VGPRs), one int8 workgroup (128 KB of LDS).
 constexpr int prefill_waves_per_simd(bool quant, int nw) { return quant ? 1 : (nw == 8 ? 4 : 2); }
 
 template <bool QUANT, int KV, int NW, int RT, int FORM>

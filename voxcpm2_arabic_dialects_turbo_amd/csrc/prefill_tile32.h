@@ -368,7 +368,10 @@ __device__ __forceinline__ void item(const PrefillArgs& p, const int qt, const i
   // One tile: the softmax of its scores (sc) beside the score MFMAs of the next tile (into sn) and its own first P V
   // MFMAs; the next V tile and the K tile after it are loaded meanwhile. In this order, pinned: an MFMA runs 32 cycles and
   // leaves the wave's issue slots free for about 1.3 elements' fma, exp, add and half a cvt, and for the LDS reads of
-  // later MFMAs (measured on one wave: 33 cycles per MFMA with that much softmax beside it, 32 without). Left to
+  // later MFMAs (a microbenchmark of one wave: 33 cycles per MFMA with that much softmax beside it, 32 without). With
+  // two waves on a SIMD the issue slots are what is short: over 16 x 2048 tokens each wave issues in 41 % of its cycles
+  // (the SIMD in 82 %), is ready behind the other in 36 % and waits in 23 %, 5 % for an LDS instruction's turn; the matrix
+  // cores are busy 53 % of the time, at a clock of 1.7 GHz, with 5.2 VALU and 1.5 LDS instructions to an MFMA. Left to
   // itself the compiler runs the MFMAs together and the softmax together, and the two waves of a SIMD do not interleave
   // the two by themselves.
   auto step = [&](int t, const f32x16 (&sc)[KT], f32x16 (&sn)[KT], const uint8_t* kn, uint8_t* kfree, const uint8_t* vc,

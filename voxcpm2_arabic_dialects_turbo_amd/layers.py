@@ -126,7 +126,7 @@ class Attention(nn.Module):
                     and _store_rides_in_prefill(k, v, context.slot_mapping):
                 # prefill: the store rides in the attention call. Over the step's own rows (no block table) the
                 # launch reads the packed rows; through the block tables (prefix cache, mixed steps) the launch reads
-                # each sequence's new keys from the rows and writes the caches after its reads
+                # each sequence's new keys from the rows, not from the cache slots it writes
                 bt = context.block_tables
                 _check_riding_store(context, k_cache.shape[1], decode=False)
                 return prefill_attention_store(q, k, v, k_cache, v_cache, context.slot_mapping,

@@ -64,7 +64,7 @@ constexpr int kMaxPieces = 32;
 constexpr int kMaxPiecesSplit = 64;
 // Batches of up to this many sequences merge with four workgroups per sequence (merge_row<4>), a quarter of the partials
 // per wave; beyond, the sequences' own workgroups fill the CUs. A layer of a step, one workgroup against four: 1 stream
-// of 420 tokens 12.0 -> 10.0 us, 13 of 2500-4096 19.9 -> 16.9, 40 of 200-1500 17.2 -> 16.1; 80 of 100-1024 18.0 -> 18.4,
+// of 420 tokens 12.0 -> 8.9 us, 13 of 2500-4096 19.9 -> 16.9, 40 of 200-1500 17.2 -> 16.1; 80 of 100-1024 18.0 -> 18.4,
 // 150 of 256-2048 37.6 -> 38.4, 256 of 50-1024 33.8 -> 35.3.
 constexpr int kMergeSplitBatch = 64;
 constexpr int kMergeBatch = VOX_MERGE_BATCH;  // partials whose loads the merge kernel keeps in flight together
